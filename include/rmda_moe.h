@@ -179,9 +179,12 @@ int rmda_moe_set_hot_rows(rmda_moe_ctx_t *ctx, uint32_t rows);
  *                       and every call after rmda_moe_set_hot_rows or this
  *                       function, runs as AUTO until its choice lands;
  *   RMDA_TILE_STREAM / RMDA_TILE_HOT  always that tile.
- * Every policy gives bitwise the same output; calls with rows < hot rows
- * (no expert can be hot) and HF-layout weights launch the streaming tile
- * only. */
+ * Under ADAPTIVE, packed-weight calls of few rows per expert or few experts
+ * run one wave per strip of 32 weight rows instead of either tile, by a rule
+ * on the shape alone (the work list is then the streaming tile's).
+ * Every policy gives bitwise the same output; other calls with rows < hot
+ * rows (no expert can be hot) and HF-layout weights launch the streaming
+ * tile only. */
 enum { RMDA_TILE_ADAPTIVE = 0, RMDA_TILE_AUTO = 1, RMDA_TILE_STREAM = 2, RMDA_TILE_HOT = 3 };
 int rmda_moe_set_tile_policy(rmda_moe_ctx_t *ctx, int policy);
 /* Route inside the rank launch for calls of more than one rank block of

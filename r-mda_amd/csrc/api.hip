@@ -1141,6 +1141,20 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // is enqueued too and does the combine only if that tile ran.
     const bool fold_combine =
         ctx->fused_combine != 0 && packed != nullptr && ctx->g2.spec != 0 && tile_mode != 2u && !x32;
+    // Few rows per expert or few experts: either GEMM may run one wave per
+    // strip of weight rows over the streaming tile's list (gemm_strip.hip).
+    // An explicit tile policy keeps its tile.
+    const uint32_t item_rows = std::min(T, RMDA_GEMM2_BM);
+    const uint32_t items_max = std::min(p.npairs, E) + p.npairs / RMDA_GEMM2_BM +
+                               (p.sh_rows + RMDA_GEMM2_BM - 1) / RMDA_GEMM2_BM;
+    const uint32_t groups = E + (p.sh_rows > 0 ? 1u : 0u);
+    const bool strip_ok = packed != nullptr && !fold_combine && ctx->tile_policy == RMDA_TILE_ADAPTIVE &&
+                          ctx->g2.spec == 6 && ((uint64_t)T * d | (uint64_t)p.groups_rows * I) < (1ull << 32);
+    const bool strip_gu = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, 2 * I, d);
+    const bool strip_dn = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, d, I);
+    if (strip_gu || strip_dn) {
+        tile_mode = 1u;
+    }
     // A2 counts, offsets, block bases and the GEMM work list
     if (rc == RMDA_OK) {
         rmda_rank_args_t ra{};
@@ -1244,7 +1258,9 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
         }
         // the compute tile first (it has work only when the rank kernel cut
         // the list for it), then the streaming tile (work only otherwise)
-        rc = gemm_pair(ctx, s, g, gu, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode, "layer gate_up");
+        rc = strip_gu ? hip_check(ctx, rmda_launch_gemm_strip(s, &g, items_max, item_rows), "layer gate_up")
+                      : gemm_pair(ctx, s, g, gu, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode,
+                                  "layer gate_up");
     }
     // x32: hp's slot-scaled fp16 cast (src/qwen.c:858-877), routed and shared rows
     if (rc == RMDA_OK && x32) {
@@ -1301,8 +1317,9 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
             g.fc.out = args->out;
             g.fc.hc = rmda_hc_t{args->h, args->inj, args->inj_stride, args->inj_off, args->hc};
         }
-        rc = gemm_pair(ctx, s, g, ctx->g2, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode,
-                       "layer down");
+        rc = strip_dn ? hip_check(ctx, rmda_launch_gemm_strip(s, &g, items_max, item_rows), "layer down")
+                      : gemm_pair(ctx, s, g, ctx->g2, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode,
+                                  "layer down");
     }
     if (rc == RMDA_OK) {
         rc = prof_mark(ctx, RMDA_STAGE_DOWN + 1);

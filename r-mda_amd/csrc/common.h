@@ -564,6 +564,15 @@ static_assert(RMDA_GEMM_HOT_BM <= 16u * RMDA_ITEM_CLASSES && RMDA_GEMM_HOT_BM <=
 // stages: LDS ring depth (4 or 5); sched: 0 = task_sched_t, 1 = chunk_sched_t
 hipError_t rmda_launch_gemm_hot(hipStream_t s, const rmda_gemm_args_t *a, uint32_t grid, int stages, int sched);
 hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm2_cfg_t c, int packed);
+// gemm_strip.hip: the same GEMMs over the same work list with one wave per
+// (64-row chunk, 32 weight rows), for calls of few rows per expert or few
+// experts (packed weights, gemm2's bits).  items bounds *n_items, item_rows
+// (<= RMDA_GEMM2_BM) the rows of an item.  32-bit offsets into A: a_rows *
+// lda, and for F16 the sorted rows * lda, below 2^32 elements.
+// rmda_gemm_strip_pays: the rule for npairs routed rows over `groups` experts
+// (shared one included).
+bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k);
+hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows);
 // Reorder `groups` row-major [n_w][k] matrices (fp16, or bf16 when bf16_in)
 // into the packed slab order of K step bk (SWIGLU: gate/up interleave).
 hipError_t rmda_launch_pack(hipStream_t s, const uint16_t *src, uint16_t *dst, uint32_t groups, uint32_t n_w,

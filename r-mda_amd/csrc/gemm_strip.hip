@@ -1,0 +1,247 @@
+// Grouped expert GEMM of the fused layer for calls of few rows per expert or
+// few experts (gfx950, packed weights).
+//
+// What bounds it.  Such a call is a weight stream: the streaming tile
+// (gemm2.hip) hands out (item, 256 weight rows) tasks of a whole workgroup
+// each, so one token of 8 selected experts is 48 gate_up and 64 down tasks on
+// 256 CUs, each waiting on its own chain of five 16 KiB stages, and a call
+// whose tasks do not fill the last round of workgroups leaves CUs idle.  Here
+// a task is one wave: a chunk of up to 64 rows of a work item times 32 weight
+// rows (a strip), 8 times as many tasks of which none waits for another.
+//   * A packed slab keeps 16 weight rows x 32 k (one MFMA operand) in one
+//     contiguous KiB, so a wave loads it straight into registers, 16 bytes
+//     per lane: no LDS and no barriers.  The weights carry the non-temporal
+//     hint.
+//   * 6 to 16 K steps (by live row groups) are in flight per wave in a
+//     register ring, within 256 VGPRs so that two waves share a SIMD: 32 MB
+//     in flight over the chip against about 3 us of loaded HBM latency.  One
+//     wave per workgroup: with 4 or 8 a finished wave's registers wait for the
+//     others (one 16-token block, hidden 2048, 128 experts top-8, width 768:
+//     gate_up 74 us, 77 and 80 us).
+//   * Activation rows are read in the MFMA layout from L2, only the live
+//     16-row groups of the chunk: the loop is specialised on their number.
+//   * The strips and chunks of one slab run on one XCD, so a chunk re-reads
+//     its weights from L2 (32 tokens of the shape above: gate_up 126 -> 102
+//     us against strips dealt round the XCDs).
+// Measured against the streaming tile on MI355X (gate_up + down, us): the
+// shape above at 1 token 33.0 + 12.8 -> 7.2 + 3.9, 16 tokens 103 + 45 -> 76
+// + 39 (6.7 TB/s), 32 tokens 116 + 60 -> 102 + 52; 256 tokens of 8 experts
+// top-2, hidden 512, width 1024: 13.2 + 19.4 -> 8.4 + 4.8.
+// Per output element the MFMA sequence and the epilogue are those of the
+// other tiles (K steps of 32 in order from a zero accumulator), so the output
+// is bitwise the same.
+#include "common.h"
+#include "gemm_sched.h"
+
+namespace {
+
+using namespace rmda_gemm;
+
+constexpr uint32_t SLAB = 256;     // packed slab height (weight rows)
+constexpr uint32_t BK = 32;        // K step of a slab block
+constexpr uint32_t STEP = SLAB * BK;
+constexpr uint32_t STRIPS = 8;     // strips of 32 weight rows in a slab
+constexpr uint32_t CHUNK = 64;     // rows of a chunk
+
+// One chunk of MT live 16-row groups times one strip.
+template <int MODE, int MT, int DEPTH, bool SC>
+__device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t row0, uint32_t rows, bool is_shared,
+                                            const uint16_t *b0, const uint16_t *b1, uint32_t col0) {
+    const uint32_t lane = threadIdx.x;
+    const uint32_t fr = lane % 16;
+    const uint32_t fq = lane / 16;
+    const uint32_t steps = g.k / BK;
+    constexpr uint32_t A_STEP = MODE == RMDA_GEMM_F16 ? RMDA_HP_ROWS * BK : BK;
+    uint32_t a[MT];  // element offsets from g.a (the launch checks that they fit)
+#pragma unroll
+    for (int m = 0; m < MT; m += 1) {
+        if (MODE == RMDA_GEMM_SWIGLU) {
+            const uint32_t r = (uint32_t)m * 16u + fr;
+            const uint32_t rr = r < rows ? r : 0u;
+            uint32_t t = is_shared ? row0 + rr - g.shared_row0 : g.rowtok[row0 + rr];
+            t = t < g.a_rows ? t : 0u;  // a bad index reads a valid row, never out of bounds
+            a[m] = t * g.lda + fq * 8;
+        } else {
+            a[m] = (uint32_t)rmda_hp_index(row0 + (uint32_t)m * 16u, 0, g.lda) + fr * 32 + fq * 8;
+        }
+    }
+    half8_t ra[DEPTH][MT], rb[DEPTH][2];
+    floatx4_t acc[MT][2];
+#pragma unroll
+    for (int m = 0; m < MT; m += 1) {
+        acc[m][0] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        acc[m][1] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    auto load = [&](uint32_t s, int u) __attribute__((always_inline)) {
+        rb[u][0] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(b0 + (size_t)s * STEP));
+        rb[u][1] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(b1 + (size_t)s * STEP));
+#pragma unroll
+        for (int m = 0; m < MT; m += 1) {
+            ra[u][m] = *reinterpret_cast<const half8_t *>(g.a + s * A_STEP + a[m]);
+        }
+    };
+    auto mma = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < MT; m += 1) {
+            acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra[u][m], rb[u][0], acc[m][0], 0, 0, 0);
+            acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra[u][m], rb[u][1], acc[m][1], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < DEPTH; u += 1) {
+        load(min((uint32_t)u, steps - 1u), u);  // past the end: a valid step, never multiplied
+    }
+    uint32_t s = 0;
+    // whole rounds whose loads all stay below `steps`
+    for (; s + 2 * DEPTH <= steps; s += DEPTH) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; u += 1) {
+            mma(u);
+            load(s + DEPTH + u, u);
+            __builtin_amdgcn_sched_barrier(0);  // as written: a slot's loads leave right after its MFMAs
+        }
+    }
+    // the last DEPTH steps, and up to DEPTH - 1 more that still need loading
+    for (; s < steps; s += DEPTH) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; u += 1) {
+            if (s + u < steps) {
+                mma(u);
+                if (s + DEPTH + u < steps) {
+                    load(s + DEPTH + u, u);
+                }
+            }
+        }
+    }
+    // the slot-scaled mode's inverse scales (1 otherwise, which changes no bits)
+    const float xinv = SC && MODE == RMDA_GEMM_SWIGLU ? rmda_slot_inv(g.xscale) : 1.0f;
+    const float yinv = down_mul<SC, MODE>(g);
+    uint16_t *const O = reinterpret_cast<uint16_t *>(g.out);
+    float hmax = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MT; m += 1) {
+#pragma unroll
+        for (int v = 0; v < 4; v += 1) {
+            const uint32_t rr = (uint32_t)m * 16u + 4 * fq + v;
+            if (rr < rows) {
+                if (MODE == RMDA_GEMM_SWIGLU) {
+                    const float h = rmda_swiglu_fast(acc[m][0][v] * xinv, acc[m][1][v] * xinv);
+                    swiglu_store<SC, false>(g, O, rmda_hp_index(row0 + rr, col0 + fr, g.ldo), h, hmax);
+                } else {
+                    const size_t o = (size_t)(row0 + rr) * g.ldo + col0 + fr;
+                    down_store<SC>(g, O, o, acc[m][0][v] * yinv);
+                    down_store<SC>(g, O, o + 16, acc[m][1][v] * yinv);
+                }
+            }
+        }
+    }
+    if (SC && MODE == RMDA_GEMM_SWIGLU) {
+        const uint32_t r = rmda_wave_red_u32<true>(__builtin_bit_cast(uint32_t, hmax));
+        if (lane == 0) {
+            atomicMax(g.hp_amax + blockIdx.x % RMDA_AMAX_PARTS * RMDA_AMAX_STRIDE, r);
+        }
+    }
+}
+
+// DEEP: 16 steps in flight for one live row group, 12 for two, 8 and 7 for
+// three and four, instead of 8, 8, 6 and 6.  It keeps HBM busy on long K
+// loops (16 tokens of the shape above: layer 149 -> 145.5 us; 512 experts
+// top-10, hidden 2560, width 640 at 512 tokens: 938 -> 915 us); a launch that
+// the shallow ring covers at once only pays for its longer start (one token:
+// 36.1 -> 37.3 us), and a K loop shorter than the ring reads its last step
+// again (K = 256: down 15.7 -> 21.0 us).
+template <int MODE, bool DEEP, bool SC>
+__global__ __launch_bounds__(RMDA_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) void strip_kernel(
+    rmda_gemm_args_t g, uint32_t chunks) {
+    const const_u32p items = (const_u32p)g.items;
+    // blockIdx.x = (slab / 8, chunk, strip, slab % 8), slabs counted over the
+    // whole work list: the strips and row chunks of a slab share an XCD's L2
+    const uint32_t nslab = g.n_w / SLAB;
+    const uint32_t j = blockIdx.x / 8u;
+    const uint32_t jj = j / STRIPS;
+    const uint32_t gs = jj / chunks * 8u + blockIdx.x % 8u;
+    const uint32_t r0 = jj % chunks * CHUNK;
+    const uint32_t item = gs / nslab;
+    const uint32_t slab = gs - item * nslab;
+    const uint32_t strip = j % STRIPS;
+    if (item >= *(const_u32p)g.n_items) {
+        return;
+    }
+    const uint32_t grp = items[item * 4 + 0];
+    const uint32_t row0 = items[item * 4 + 1] + r0;
+    const uint32_t n = items[item * 4 + 2];
+    if (r0 >= n) {
+        return;
+    }
+    const uint32_t rows = min(n - r0, CHUNK);
+    const uint32_t fr = threadIdx.x % 16;
+    const uint32_t fq = threadIdx.x / 16;
+    const bool is_shared = grp == g.shared_group;
+    const uint16_t *const wg = is_shared ? g.w_shared : g.w + (size_t)grp * g.n_w * g.k;
+    // weight rows of the strip: two 16-row operands.  SWIGLU: 16 gate rows
+    // and the matching up rows, 32 slab rows further; F16: 32 adjacent rows
+    const uint32_t nb = MODE == RMDA_GEMM_SWIGLU ? strip / 2u * 64u + strip % 2u * 16u : strip * 32u;
+    const uint32_t col0 = MODE == RMDA_GEMM_SWIGLU ? slab * (SLAB / 2) + strip * 16u : slab * SLAB + strip * 32u;
+    const uint16_t *const b0 =
+        wg + (size_t)slab * (g.k / BK) * STEP + nb * BK + fr * BK + (fq ^ swz<BK>(fr)) * 8;
+    const uint16_t *const b1 = b0 + (MODE == RMDA_GEMM_SWIGLU ? 32u : 16u) * BK;
+    switch ((rows + 15u) / 16u) {
+    case 1: strip_chunk<MODE, 1, DEEP ? 16 : 8, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
+    case 2: strip_chunk<MODE, 2, DEEP ? 12 : 8, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
+    case 3: strip_chunk<MODE, 3, DEEP ? 8 : 6, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
+    default: strip_chunk<MODE, 4, DEEP ? 7 : 6, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
+    }
+}
+
+template <int MODE, bool DEEP>
+hipError_t launch_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
+    const uint32_t chunks = (item_rows + CHUNK - 1) / CHUNK;
+    const dim3 grid((items * (a->n_w / SLAB) + 7) / 8 * 8 * STRIPS * chunks);
+    const bool sc = a->hp32 != nullptr || a->ye_bound != nullptr;
+    if (sc) {
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, true>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+    } else {
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k) {
+    const uint64_t tasks = (uint64_t)items * (n_w / SLAB);  // the streaming tile's
+    // Experts average few rows: every strip is read once and the weights
+    // decide.  Up to 4 rows where the streaming tile's tasks fill two rounds
+    // of the 256 workgroups (128 experts of width 768: 4 rows, layer 210 ->
+    // 204 us; 8 rows, 215 -> 213 us but 85 -> 91 us under skewed routing; 16
+    // rows, 225 -> 244 us), and the more the emptier its rounds are (128
+    // tasks: 16 rows, 82 -> 69 us; 32 rows, 94 -> 118 us).
+    if ((uint64_t)npairs * (tasks < 512 ? tasks : 512) <= 4ull * 512 * groups) {
+        return true;
+    }
+    // Few weights for the streaming tile's workgroups: one round or less of
+    // tasks, and with the 64-row chunks counted at most 64 MB moved from L2 (8 experts, hidden 512, width 1024: 64
+    // rows per expert 51 -> 34 us, 128 rows 60 -> 42 us, 256 rows' gate_up,
+    // 75 MB, 18.9 -> 27.9 us; 288 tasks of hidden 768, width 256 at 80
+    // skewed rows: layer 63 -> 65 us).
+    const uint64_t bytes = 2ull * groups * n_w * k;
+    return tasks <= 256 && bytes * ((uint64_t)npairs + 32ull * groups) / (64ull * groups) <= (64ull << 20);
+}
+
+hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
+    if (a->n_w % SLAB != 0 || a->k % BK != 0 || a->n_items == nullptr || a->fc.cnt != nullptr || a->ye32 != nullptr) {
+        return hipErrorInvalidValue;
+    }
+    if (items == 0 || item_rows == 0) {
+        return hipSuccess;
+    }
+    // more waves than the chip holds at once (two per SIMD), and a K loop that
+    // fills the deep ring
+    const bool deep = (uint64_t)items * (a->n_w / 32u) > 2048 && a->k >= 16 * BK;
+    if (a->mode == RMDA_GEMM_SWIGLU) {
+        return deep ? launch_strip<RMDA_GEMM_SWIGLU, true>(s, a, items, item_rows)
+                    : launch_strip<RMDA_GEMM_SWIGLU, false>(s, a, items, item_rows);
+    }
+    return deep ? launch_strip<RMDA_GEMM_F16, true>(s, a, items, item_rows)
+                : launch_strip<RMDA_GEMM_F16, false>(s, a, items, item_rows);
+}
