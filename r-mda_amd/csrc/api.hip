@@ -1408,42 +1408,24 @@ int pack_layer(rmda_moe_ctx_t *ctx, hipStream_t s, const rmda_moe_shape_t *shape
                const uint16_t *gu, int gu_bf16, const uint16_t *dn, int dn_bf16, const uint16_t *sgu, int sgu_bf16,
                const uint16_t *sdn, int sdn_bf16, uint16_t *packed) {
     const PackPlan pk = plan_pack(shape);
-    const uint32_t E = shape->experts, d = shape->d, I = shape->inter, S = shape->shared;
-    const int bk = (int)ctx->g2.bk;
-    int rc = hip_check(ctx, rmda_launch_pack(s, gu, packed + pk.gate_up, E, 2 * I, d, I, 1, bk, gu_bf16),
-                       "pack gate_up");
-    if (rc == RMDA_OK) {
-        rc = hip_check(ctx, rmda_launch_pack(s, dn, packed + pk.down, E, d, I, I, 0, bk, dn_bf16), "pack down");
+    const uint32_t E = shape->experts, S = shape->shared;
+    rmda_pack_args_t a{};
+    a.experts = E;
+    a.d = shape->d;
+    a.inter = shape->inter;
+    a.gate_up = rmda_pack_mat_t{gu, packed + pk.gate_up, gu_bf16};
+    a.down = rmda_pack_mat_t{dn, packed + pk.down, dn_bf16};
+    if (S > 0) {
+        a.sh_gate_up = rmda_pack_mat_t{sgu, packed + pk.sh_gate_up, sgu_bf16};
+        a.sh_down = rmda_pack_mat_t{sdn, packed + pk.sh_down, sdn_bf16};
     }
-    if (rc == RMDA_OK && S > 0) {
-        rc = hip_check(ctx, rmda_launch_pack(s, sgu, packed + pk.sh_gate_up, 1, 2 * S, d, S, 1, bk, sgu_bf16),
-                       "pack shared gate_up");
-    }
-    if (rc == RMDA_OK && S > 0) {
-        rc = hip_check(ctx, rmda_launch_pack(s, sdn, packed + pk.sh_down, 1, d, S, S, 0, bk, sdn_bf16),
-                       "pack shared down");
-    }
-    if (rc == RMDA_OK) {
-        rc = hip_check(ctx,
-                       rmda_launch_router_pack(s, w_router, reinterpret_cast<float *>(packed + pk.router),
-                                               E + (S > 0 ? 1u : 0u), d),
-                       "pack router");
-    }
-    // the largest row sum of |w| over the packed down weights (routed and
-    // shared), which sizes the slot-scaled mode's fp16 expert rows; the rest
-    // of its 256 bytes is zero, so equal weights pack to equal buffers
-    uint32_t *bound = reinterpret_cast<uint32_t *>(packed + pk.bound);
-    if (rc == RMDA_OK) {
-        rc = hip_check(ctx, rmda_launch_zero(s, bound, 64, 0), "pack bound fill");
-    }
-    if (rc == RMDA_OK) {
-        rc = hip_check(ctx, rmda_launch_row_abs_max(s, packed + pk.down, E, d, I, bk, bound), "pack down bound");
-    }
-    if (rc == RMDA_OK && S > 0) {
-        rc = hip_check(ctx, rmda_launch_row_abs_max(s, packed + pk.sh_down, 1, d, S, bk, bound),
-                       "pack shared down bound");
-    }
-    return rc;
+    a.w_router = w_router;
+    a.router = reinterpret_cast<float *>(packed + pk.router);
+    a.router_cols = E + (S > 0 ? 1u : 0u);
+    // the bound sizes the slot-scaled mode's fp16 expert rows; the rest of
+    // its 256 bytes is zero, so equal weights pack to equal buffers
+    a.bound = reinterpret_cast<uint32_t *>(packed + pk.bound);
+    return hip_check(ctx, rmda_launch_pack(s, &a), "pack");
 }
 
 }  // namespace

@@ -323,7 +323,22 @@ hipError_t rmda_launch_router(hipStream_t s, const uint16_t *x16, const float *w
                               const rmda_route_fuse_t *fuse, const uint32_t *xscale = nullptr);
 // Packed router weights: [d/16][rmda_router_cpad(cols)][4][4] fp32, element
 // (k, c) at ((k/16)*cpad + c)*16 + (k%4)*4 + (k%16)/4.
-uint32_t rmda_router_cpad(uint32_t cols);
+__host__ __device__ __forceinline__ uint32_t rmda_router_cpad(uint32_t cols) {
+    return (cols + RMDA_WAVE - 1) / RMDA_WAVE * RMDA_WAVE;
+}
+// Block b of nb's share of the router packing (256 threads), zero columns
+// past `cols`.
+__device__ __forceinline__ void rmda_router_pack_share(const float *__restrict__ w, float *__restrict__ out,
+                                                       uint32_t cols, uint32_t d, uint32_t b, uint32_t nb) {
+    const uint32_t cpad = rmda_router_cpad(cols);
+    const size_t n = (size_t)d * cpad;
+    for (size_t o = (size_t)b * 256 + threadIdx.x; o < n; o += (size_t)nb * 256) {
+        const uint32_t j = (uint32_t)(o % 16);
+        const uint32_t c = (uint32_t)((o / 16) % cpad);
+        const uint32_t k = (uint32_t)(o / (16 * (size_t)cpad)) * 16 + (j % 4) * 4 + j / 4;
+        out[o] = c < cols ? w[(size_t)c * d + k] : 0.0f;
+    }
+}
 hipError_t rmda_launch_router_pack(hipStream_t s, const float *w, float *out, uint32_t cols, uint32_t d);
 
 // route.hip: top-k per row; count gets atomic adds (caller zeroes it first).
@@ -573,15 +588,31 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
 // (shared one included).
 bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k);
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows);
-// Reorder `groups` row-major [n_w][k] matrices (fp16, or bf16 when bf16_in)
-// into the packed slab order of K step bk (SWIGLU: gate/up interleave).
-hipError_t rmda_launch_pack(hipStream_t s, const uint16_t *src, uint16_t *dst, uint32_t groups, uint32_t n_w,
-                            uint32_t k, uint32_t inter, int swiglu, int bk, int bf16_in);
-// The largest row sum of |w| over `groups` packed (non-SwiGLU) matrices
-// [n_w][k] of K step bk, rows whose sum is not finite left out, atomicMax'ed
-// as float bits into *bound (which the caller zeroes first).
-hipError_t rmda_launch_row_abs_max(hipStream_t s, const uint16_t *packed, uint32_t groups, uint32_t n_w, uint32_t k,
-                                   int bk, uint32_t *bound);
+// Packed slab height: weight rows of one N tile (256 of gate_up's 2 * inter,
+// or of down's d).
+#define RMDA_SLAB 256u
+// pack.hip: one layer's weights into the packed order, two launches: gate_up
+// (routed, shared), the router rows and the cleared bound word; then down
+// (routed, shared) with the bound.  Packed slab image: for slab t and K step
+// ks of 32, 16-byte unit (n, p) holds W[slab_row(t, n)][ks*32 + (p ^
+// swz(n))*8 .. +8], at unit index ((t * steps + ks) * 256 + n) * 4 + p.  The
+// bound is the largest row sum of |w| over the packed down weights, rows
+// whose sum is not finite left out, as float bits; each row is summed in
+// packed order.
+struct rmda_pack_mat_t {
+    const uint16_t *src;
+    uint16_t *dst;
+    int bf16;  // src is bf16, converted to fp16 (round to nearest even)
+};
+struct rmda_pack_args_t {
+    uint32_t experts, d, inter;
+    rmda_pack_mat_t gate_up, sh_gate_up, down, sh_down;  // shared: src NULL when there is none (its width is inter)
+    const float *w_router;
+    float *router;
+    uint32_t router_cols;
+    uint32_t *bound;  // 64 words: the bound, then zeros
+};
+hipError_t rmda_launch_pack(hipStream_t s, const rmda_pack_args_t *a);
 
 // combine.hip
 hipError_t rmda_launch_combine(hipStream_t s, const rmda_pc_moe_combine_t *pc, const float *wt,

@@ -1,6 +1,5 @@
 // Grouped expert GEMM of the fused layer: weight-streaming design for gfx950.
-// Serves the gate_up GEMM (SwiGLU epilogue) and the down GEMM, and packs the
-// expert weights into the order it streams them.
+// Serves the gate_up GEMM (SwiGLU epilogue) and the down GEMM.
 //
 // Why this shape.  At the benchmark shapes every expert's weight slice is
 // needed by ~128 token rows, so the GEMM is bound by streaming the weights
@@ -68,22 +67,7 @@ namespace {
 using namespace rmda_gemm;
 
 constexpr uint32_t BM = RMDA_GEMM2_BM;  // rows per work item (three 64-row blocks)
-constexpr uint32_t SLAB = 256;          // packed slab height (B rows) = the N tile
-
-// B row of a group's weight matrix that slab row n of slab `slab` holds.
-// A SWIGLU slab is SLAB/64 groups of 32 gate rows followed by the 32
-// matching up rows, so one wave's accumulators hold gate and up of the same
-// output columns.
-template <int MODE>
-__device__ __forceinline__ uint32_t slab_row(uint32_t slab, uint32_t n, uint32_t inter) {
-    if (MODE == RMDA_GEMM_SWIGLU) {
-        const uint32_t bw = n / 64;
-        const uint32_t within = n % 64;
-        const uint32_t c = slab * (SLAB / 2) + bw * 32 + (within % 32);
-        return within < 32 ? c : inter + c;
-    }
-    return slab * SLAB + n;
-}
+constexpr uint32_t SLAB = RMDA_SLAB;    // packed slab height (B rows) = the N tile
 
 // Persistent workgroup: MB (=3) blocks of 64 rows x BN/64 (=4) column
 // blocks of 64, one wave each (12 waves).  Waves w and w + 4 share a SIMD, so
@@ -1139,83 +1123,6 @@ __global__ __launch_bounds__(1024) void gemm4_kernel(rmda_gemm_args_t g) {
     }
 }
 
-// Packed slab image: for slab t (128 B rows) and K step ks, 16-byte unit
-// (n, p) holds B[slab_row(t, n)][ks*BK + (p ^ swz(n))*8 .. +8], at unit
-// index ((t * steps + ks) * 128 + n) * (BK/8) + p.
-template <int MODE, int BK>
-__global__ __launch_bounds__(256) void pack_kernel(const uint16_t *__restrict__ src, uint16_t *__restrict__ dst,
-                                                   uint32_t groups, uint32_t n_w, uint32_t k, uint32_t inter,
-                                                   int bf16_in) {
-    constexpr uint32_t CH = BK / 8;
-    const uint64_t per_group = (uint64_t)n_w * k / 8;  // 16-byte units
-    const uint64_t total = per_group * groups;
-    const uint32_t steps = k / BK;
-    for (uint64_t u = (uint64_t)blockIdx.x * 256 + threadIdx.x; u < total; u += (uint64_t)gridDim.x * 256) {
-        const uint64_t gi = u / per_group;
-        const uint64_t r = u % per_group;
-        const uint32_t p = (uint32_t)(r % CH);
-        const uint32_t n = (uint32_t)((r / CH) % SLAB);
-        const uint64_t ts = r / (CH * SLAB);
-        const uint32_t ks = (uint32_t)(ts % steps);
-        const uint32_t t = (uint32_t)(ts / steps);
-        const uint32_t row = slab_row<MODE>(t, n, inter);
-        const uint32_t col = ks * BK + (p ^ swz<BK>(n)) * 8;
-        const uint4 v = *reinterpret_cast<const uint4 *>(src + (gi * n_w + row) * k + col);
-        uint4 o = v;
-        if (bf16_in) {
-            const uint32_t in[4] = {v.x, v.y, v.z, v.w};
-            uint32_t out[4];
-#pragma unroll
-            for (int q = 0; q < 4; q += 1) {
-                const float lo = __builtin_bit_cast(float, in[q] << 16);
-                const float hi = __builtin_bit_cast(float, in[q] & 0xffff0000u);
-                out[q] = (uint32_t)rmda_f2h(lo) | ((uint32_t)rmda_f2h(hi) << 16);
-            }
-            o = make_uint4(out[0], out[1], out[2], out[3]);
-        }
-        reinterpret_cast<uint4 *>(dst)[u] = o;
-    }
-}
-
-// The largest row sum of |w| over `groups` packed F16-mode matrices [n_w][k]
-// (the down weights; one thread per weight row, its slab row's 64 bytes per
-// K step, so a wave reads whole lines), rows whose sum is not finite left
-// out, as float bits: a wave maximum, then one atomicMax per wave.
-template <int BK>
-__global__ __launch_bounds__(256) void row_abs_kernel(const uint16_t *__restrict__ packed, uint32_t groups,
-                                                      uint32_t n_w, uint32_t k, uint32_t *__restrict__ bound) {
-    constexpr uint32_t CH = BK / 8;
-    const uint32_t steps = k / BK;
-    const uint64_t rows = (uint64_t)groups * n_w;
-    const uint4 *units = reinterpret_cast<const uint4 *>(packed);
-    float m = 0.0f;
-    for (uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x; q < rows; q += (uint64_t)gridDim.x * 256) {
-        const uint64_t gi = q / n_w;
-        const uint32_t r = (uint32_t)(q % n_w);
-        // unit (gi, t, ks, n, p) = gi * n_w * k / 8 + ((t * steps + ks) * SLAB + n) * CH + p
-        const uint4 *u = units + gi * n_w * k / 8 + ((uint64_t)(r / SLAB) * steps * SLAB + r % SLAB) * CH;
-        float sum = 0.0f;
-        for (uint32_t ks = 0; ks < steps; ks += 1) {
-#pragma unroll
-            for (uint32_t p = 0; p < CH; p += 1) {
-                const uint4 v = u[(size_t)ks * SLAB * CH + p];
-                const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int i = 0; i < 4; i += 1) {
-                    sum += fabsf(rmda_h2f((uint16_t)(w4[i] & 0xffffu))) + fabsf(rmda_h2f((uint16_t)(w4[i] >> 16)));
-                }
-            }
-        }
-        if (sum <= 3.4028235e38f) {  // false for inf and NaN
-            m = fmaxf(m, sum);
-        }
-    }
-    const uint32_t b = rmda_wave_red_u32<true>(__builtin_bit_cast(uint32_t, m));
-    if (threadIdx.x % RMDA_WAVE == 0) {
-        atomicMax(bound, b);
-    }
-}
-
 template <int MODE, int BN, int BK, int STAGES, int BPOL, bool SC = false>
 hipError_t launch_cfg(hipStream_t s, const rmda_gemm_args_t *a, dim3 grid, bool packed) {
     if (packed) {
@@ -1330,56 +1237,4 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
         return launch_mode<RMDA_GEMM_SWIGLU>(s, a, c, packed != 0);
     }
     return launch_mode<RMDA_GEMM_F16>(s, a, c, packed != 0);
-}
-
-hipError_t rmda_launch_row_abs_max(hipStream_t s, const uint16_t *packed, uint32_t groups, uint32_t n_w, uint32_t k,
-                                   int bk, uint32_t *bound) {
-    const uint64_t rows = (uint64_t)groups * n_w;
-    if (rows == 0) {
-        return hipSuccess;
-    }
-    if (n_w % SLAB != 0 || k % bk != 0 || (bk != 32 && bk != 64)) {
-        return hipErrorInvalidValue;
-    }
-    const dim3 grid((uint32_t)std::min<uint64_t>((rows + 255) / 256, 4096));
-    if (bk == 64) {
-        hipLaunchKernelGGL(row_abs_kernel<64>, grid, dim3(256), 0, s, packed, groups, n_w, k, bound);
-    } else {
-        hipLaunchKernelGGL(row_abs_kernel<32>, grid, dim3(256), 0, s, packed, groups, n_w, k, bound);
-    }
-    return hipGetLastError();
-}
-
-hipError_t rmda_launch_pack(hipStream_t s, const uint16_t *src, uint16_t *dst, uint32_t groups, uint32_t n_w,
-                            uint32_t k, uint32_t inter, int swiglu, int bk, int bf16_in) {
-    const uint64_t units = (uint64_t)groups * n_w * k / 8;
-    if (units == 0) {
-        return hipSuccess;
-    }
-    if (n_w % SLAB != 0 || k % bk != 0) {
-        return hipErrorInvalidValue;
-    }
-    uint64_t blocks = (units + 255) / 256;
-    if (blocks > 16384) {
-        blocks = 16384;
-    }
-    const dim3 grid((uint32_t)blocks);
-    if (swiglu) {
-        if (bk == 64) {
-            hipLaunchKernelGGL((pack_kernel<RMDA_GEMM_SWIGLU, 64>), grid, dim3(256), 0, s, src, dst, groups, n_w, k,
-                               inter, bf16_in);
-        } else {
-            hipLaunchKernelGGL((pack_kernel<RMDA_GEMM_SWIGLU, 32>), grid, dim3(256), 0, s, src, dst, groups, n_w, k,
-                               inter, bf16_in);
-        }
-    } else {
-        if (bk == 64) {
-            hipLaunchKernelGGL((pack_kernel<RMDA_GEMM_F16, 64>), grid, dim3(256), 0, s, src, dst, groups, n_w, k,
-                               inter, bf16_in);
-        } else {
-            hipLaunchKernelGGL((pack_kernel<RMDA_GEMM_F16, 32>), grid, dim3(256), 0, s, src, dst, groups, n_w, k,
-                               inter, bf16_in);
-        }
-    }
-    return hipGetLastError();
 }

@@ -20,6 +20,21 @@ __device__ __forceinline__ uint32_t swz(uint32_t r) {
     return (r >> 1) & (uint32_t)(BK / 8 - 1);
 }
 
+// B row of a group's weight matrix that slab row n of slab `slab` holds.
+// A SWIGLU slab is RMDA_SLAB/64 groups of 32 gate rows followed by the 32
+// matching up rows, so one wave's accumulators hold gate and up of the same
+// output columns.
+template <int MODE>
+__device__ __forceinline__ uint32_t slab_row(uint32_t slab, uint32_t n, uint32_t inter) {
+    if (MODE == RMDA_GEMM_SWIGLU) {
+        const uint32_t bw = n / 64;
+        const uint32_t within = n % 64;
+        const uint32_t c = slab * (RMDA_SLAB / 2) + bw * 32 + (within % 32);
+        return within < 32 ? c : inter + c;
+    }
+    return slab * RMDA_SLAB + n;
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

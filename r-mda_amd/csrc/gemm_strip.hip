@@ -37,7 +37,7 @@ namespace {
 
 using namespace rmda_gemm;
 
-constexpr uint32_t SLAB = 256;     // packed slab height (weight rows)
+constexpr uint32_t SLAB = RMDA_SLAB;
 constexpr uint32_t BK = 32;        // K step of a slab block
 constexpr uint32_t STEP = SLAB * BK;
 constexpr uint32_t STRIPS = 8;     // strips of 32 weight rows in a slab

@@ -640,23 +640,13 @@ __global__ __launch_bounds__(RW_NT) void router_wide_kernel(const uint16_t *__re
     }
 }
 
-// HF router weights [cols][d] -> packed [d/16][cpad][4][4]: element (k, c)
-// at ((k/16)*cpad + c)*16 + (k%4)*4 + (k%16)/4, zero columns past `cols`.
-// One thread per packed float; a one-time load-time reorder.
+// HF router weights [cols][d] -> packed, a load-time reorder
 __global__ __launch_bounds__(256) void router_pack_kernel(const float *__restrict__ w, float *__restrict__ out,
-                                                          uint32_t cols, uint32_t cpad, uint32_t d) {
-    const size_t n = (size_t)d * cpad;
-    for (size_t o = (size_t)blockIdx.x * 256 + threadIdx.x; o < n; o += (size_t)gridDim.x * 256) {
-        const uint32_t j = (uint32_t)(o % 16);
-        const uint32_t c = (uint32_t)((o / 16) % cpad);
-        const uint32_t k = (uint32_t)(o / (16 * (size_t)cpad)) * 16 + (j % 4) * 4 + j / 4;
-        out[o] = c < cols ? w[(size_t)c * d + k] : 0.0f;
-    }
+                                                          uint32_t cols, uint32_t d) {
+    rmda_router_pack_share(w, out, cols, d, blockIdx.x, gridDim.x);
 }
 
 }  // namespace
-
-uint32_t rmda_router_cpad(uint32_t cols) { return (cols + RMDA_WAVE - 1) / RMDA_WAVE * RMDA_WAVE; }
 
 namespace {
 
@@ -761,6 +751,6 @@ hipError_t rmda_launch_router_pack(hipStream_t s, const float *w, float *out, ui
     const uint32_t cpad = rmda_router_cpad(cols);
     const size_t n = (size_t)d * cpad;
     const uint32_t blocks = (uint32_t)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
-    hipLaunchKernelGGL(router_pack_kernel, dim3(blocks > 0 ? blocks : 1), dim3(256), 0, s, w, out, cols, cpad, d);
+    hipLaunchKernelGGL(router_pack_kernel, dim3(blocks > 0 ? blocks : 1), dim3(256), 0, s, w, out, cols, d);
     return hipGetLastError();
 }
