@@ -1122,10 +1122,22 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     } else if (rc == RMDA_OK) {
         prof_skip(ctx, RMDA_STAGE_ROUTE);
     }
+    // Few rows per expert or few experts: either GEMM may run one wave per
+    // strip of weight rows over the streaming tile's list (gemm_strip.hip).
+    // An explicit tile policy keeps its tile.
+    const uint32_t item_rows = std::min(T, RMDA_GEMM2_BM);
+    const uint32_t items_max = std::min(p.npairs, E) + p.npairs / RMDA_GEMM2_BM +
+                               (p.sh_rows + RMDA_GEMM2_BM - 1) / RMDA_GEMM2_BM;
+    const uint32_t groups = E + (p.sh_rows > 0 ? 1u : 0u);
+    const bool strip_ok = packed != nullptr && ctx->fused_combine == 0 && ctx->tile_policy == RMDA_TILE_ADAPTIVE &&
+                          ctx->g2.spec == 6 && ((uint64_t)T * d | (uint64_t)p.groups_rows * I) < (1ull << 32);
+    const bool strip_gu = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, 2 * I, d);
+    const bool strip_dn = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, d, I);
     // Tile of the two GEMMs (0: both launch, the rank kernel decides; 1: the
     // streaming tile only; 2: the compute tile only).  No expert can be hot
     // with fewer rows than hot_min (a token adds at most one row per expert).
-    const bool hot_possible = packed != nullptr && ctx->hot_min > 0 && T >= ctx->hot_min;
+    const bool hot_possible =
+        packed != nullptr && ctx->hot_min > 0 && T >= ctx->hot_min && !strip_gu && !strip_dn;
     uint32_t tile_mode = 1;
     uint32_t hint_slot = 0;
     if (hot_possible) {
@@ -1141,20 +1153,6 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // is enqueued too and does the combine only if that tile ran.
     const bool fold_combine =
         ctx->fused_combine != 0 && packed != nullptr && ctx->g2.spec != 0 && tile_mode != 2u && !x32;
-    // Few rows per expert or few experts: either GEMM may run one wave per
-    // strip of weight rows over the streaming tile's list (gemm_strip.hip).
-    // An explicit tile policy keeps its tile.
-    const uint32_t item_rows = std::min(T, RMDA_GEMM2_BM);
-    const uint32_t items_max = std::min(p.npairs, E) + p.npairs / RMDA_GEMM2_BM +
-                               (p.sh_rows + RMDA_GEMM2_BM - 1) / RMDA_GEMM2_BM;
-    const uint32_t groups = E + (p.sh_rows > 0 ? 1u : 0u);
-    const bool strip_ok = packed != nullptr && !fold_combine && ctx->tile_policy == RMDA_TILE_ADAPTIVE &&
-                          ctx->g2.spec == 6 && ((uint64_t)T * d | (uint64_t)p.groups_rows * I) < (1ull << 32);
-    const bool strip_gu = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, 2 * I, d);
-    const bool strip_dn = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, d, I);
-    if (strip_gu || strip_dn) {
-        tile_mode = 1u;
-    }
     // A2 counts, offsets, block bases and the GEMM work list
     if (rc == RMDA_OK) {
         rmda_rank_args_t ra{};

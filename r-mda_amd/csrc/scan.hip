@@ -637,6 +637,145 @@ __global__ __launch_bounds__(NT) void rank_kernel(rmda_rank_args_t a) {
     }
 }
 
+// Rank launch of a call of at most RMDA_RANK_BLOCK pairs whose work list is
+// the streaming tile's: one workgroup, one thread per pair.  NV > 0: the top-k
+// folded in, for up to RANK1_ROUTE_ROWS rows.
+//
+// What bounds it: latency, a chain of barriers and memory round trips.
+// Against rank_kernel it ranks all pairs in one pass over per-group lane
+// masks (rank_kernel's block of 256 threads takes four, with three barriers
+// each), and with the top-k folded in the selections go from the routing
+// waves to the ranking threads through LDS, where rank_kernel's blocks hand
+// them over through a device-scope ticket.  Measured on MI355X by events,
+// net of the empty interval: 1 token of 128 experts 6.5 -> 3.7 us, 16 tokens
+// of 512 experts top-10 9.0 -> 7.9 us, 512 pairs routed by the router kernel
+// 4.3 -> 2.1 us.  More rows than waves go to rank_kernel, whose blocks route
+// on several CUs (32 tokens of 512 experts: 9.4 us there, 14.3 us here).
+constexpr uint32_t RANK1_NT = 1024;
+constexpr uint32_t RANK1_GROUPS = RMDA_RANK_BLOCK / RMDA_WAVE;
+constexpr uint32_t RANK1_ROUTE_ROWS = RANK1_NT / RMDA_WAVE;  // one per wave
+
+template <int NV>
+__global__ __launch_bounds__(RANK1_NT) void rank1_kernel(rmda_rank_args_t a) {
+    __shared__ unsigned long long msk[RANK1_GROUPS][RMDA_MAX_EXPERTS];  // lanes of a 64-pair group by expert
+    __shared__ uint32_t sel[NV > 0 ? RMDA_RANK_BLOCK : 1];
+    __shared__ uint32_t offs[RMDA_MAX_EXPERTS];
+    __shared__ uint32_t sbuf[RANK1_NT / RMDA_WAVE];
+    __shared__ uint32_t cls_n[RMDA_ITEM_CLASSES];
+    __shared__ uint32_t cls_b[RMDA_ITEM_CLASSES];
+    __shared__ uint32_t sh_slot[2];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid % RMDA_WAVE;
+    const uint32_t w = tid / RMDA_WAVE;
+    const uint32_t E = a.experts;
+    const uint32_t groups = (a.npairs + RMDA_WAVE - 1u) / RMDA_WAVE;
+    const bool pair = tid < a.npairs;
+    uint32_t e = RMDA_NONE;
+    if (NV == 0 && pair) {
+        e = a.idx[tid];
+    }
+    for (uint32_t g = w; g < groups; g += RANK1_NT / RMDA_WAVE) {
+        for (uint32_t i = lane; i < E; i += RMDA_WAVE) {
+            msk[g][i] = 0ull;
+        }
+    }
+    if (tid < RMDA_ITEM_CLASSES) {
+        cls_n[tid] = 0;
+    }
+    if constexpr (NV > 0) {
+        if (w < a.route_rows) {
+            float v[NV];
+            rmda_route_load<NV, false>(a.route_proj + (size_t)w * a.route_stride, E, v);
+            rmda_route_select<NV>(v, a.topk, a.route_idx + (size_t)w * a.topk, a.route_wt + (size_t)w * a.topk, nullptr,
+                                  sel + w * a.topk);
+        }
+    }
+    __syncthreads();
+    if (NV > 0 && pair) {
+        e = sel[tid];
+    }
+    const bool live = e < E;  // false for RMDA_NONE and past the last pair
+    if (live) {
+        atomicOr(&msk[w][e], 1ull << lane);
+    }
+    __syncthreads();
+    uint32_t r = 0;
+    if (live) {
+        for (uint32_t g = 0; g < w; g += 1) {
+            r += __popcll(msk[g][e]);
+        }
+        r += __popcll(msk[w][e] & ((1ull << lane) - 1ull));
+    }
+    uint32_t c = 0;  // thread i < E: expert i's rows
+    if (tid < E) {
+        for (uint32_t g = 0; g < groups; g += 1) {
+            c += __popcll(msk[g][tid]);
+        }
+    }
+    uint32_t total;
+    const uint32_t o = block_exscan<RANK1_NT>((c + a.tile - 1u) / a.tile * a.tile, sbuf, &total);
+    if (tid < E) {
+        a.off[tid] = o;
+        a.count[tid] = c;
+        offs[tid] = o;
+    }
+    // work list: as rank_kernel's, sorted by rows in 16-row classes
+    const uint32_t bm = a.bm;
+    const uint32_t ncls = (bm + 15u) / 16u;
+    const uint32_t ni = (c + bm - 1u) / bm;
+    const uint32_t nfull = ni > 0 ? ni - 1u : 0u;
+    const uint32_t last_cls = ni > 0 ? (c - nfull * bm + 15u) / 16u : 0u;
+    uint32_t slot_full = 0;
+    uint32_t slot_last = 0;
+    if (nfull > 0) {
+        slot_full = atomicAdd(&cls_n[ncls - 1u], nfull);
+    }
+    if (ni > 0) {
+        slot_last = atomicAdd(&cls_n[last_cls - 1u], 1u);
+    }
+    const uint32_t ns = (a.shared_rows + bm - 1u) / bm;
+    if (tid == 0 && ns > 0) {
+        sh_slot[0] = ns > 1 ? atomicAdd(&cls_n[ncls - 1u], ns - 1u) : 0u;
+        sh_slot[1] = atomicAdd(&cls_n[(a.shared_rows - (ns - 1u) * bm + 15u) / 16u - 1u], 1u);
+    }
+    __syncthreads();
+    if (tid < ncls) {  // the items of the larger classes come first
+        uint32_t base = 0;
+        for (uint32_t q = tid + 1u; q < ncls; q += 1) {
+            base += cls_n[q];
+        }
+        cls_b[tid] = base;
+        if (tid == 0) {
+            *a.n_items = base + cls_n[0];
+            if (a.n_items_hot != nullptr) {
+                *a.n_items_hot = 0u;
+            }
+        }
+    }
+    if (pair) {
+        const uint32_t sl = live ? offs[e] + r : RMDA_NONE;
+        a.slot[tid] = sl;
+        if (live) {
+            a.rowtok[sl] = tid / a.topk;
+        }
+    }
+    __syncthreads();
+    uint4 *items = reinterpret_cast<uint4 *>(a.items);
+    for (uint32_t i = 0; i < nfull; i += 1) {
+        items[cls_b[ncls - 1u] + slot_full + i] = make_uint4(tid, o + i * bm, bm, 0u);
+    }
+    if (ni > 0) {
+        items[cls_b[last_cls - 1u] + slot_last] = make_uint4(tid, o + nfull * bm, c - nfull * bm, 0u);
+    }
+    for (uint32_t i = tid; i + 1u < ns; i += RANK1_NT) {
+        items[cls_b[ncls - 1u] + sh_slot[0] + i] = make_uint4(E, a.shared_row0 + i * bm, bm, 0u);
+    }
+    if (tid == 0 && ns > 0) {
+        const uint32_t rows = a.shared_rows - (ns - 1u) * bm;
+        items[cls_b[(rows + 15u) / 16u - 1u] + sh_slot[1]] = make_uint4(E, a.shared_row0 + (ns - 1u) * bm, rows, 0u);
+    }
+}
+
 // count[e] = number of idx[0, npairs) equal to e, for up to
 // RMDA_COUNT1_MAX_PAIRS pairs: one 1024-thread block, an LDS histogram, no
 // hand-off between blocks.  Four 16-byte loads per thread in flight when idx
@@ -748,6 +887,27 @@ hipError_t rmda_launch_rank(hipStream_t s, const rmda_rank_args_t *a) {
     uint32_t nb = (a->npairs + RMDA_RANK_BLOCK - 1) / RMDA_RANK_BLOCK;
     if (nb == 0) {
         nb = 1;  // one block still finalises (zero counts, empty work list)
+    }
+    // one rank block, a streaming-tile list, at most RANK1_ROUTE_ROWS rows to
+    // route: the one-workgroup kernel
+    const bool rank1 = nb == 1 && a->items != nullptr && a->slot != nullptr && a->rowtok != nullptr &&
+                       a->off != nullptr && a->count != nullptr && a->off_in == nullptr && a->fc_cnt == nullptr &&
+                       a->hint_out == nullptr && (a->hot_min == 0 || a->force == 1u) && a->force != 2u &&
+                       (a->route_proj == nullptr ||
+                        (a->route_rows <= RANK1_ROUTE_ROWS && a->route_rows * a->topk == a->npairs));
+    if (rank1) {
+        const uint32_t nv = a->route_proj == nullptr ? 0u : (a->experts + RMDA_WAVE - 1) / RMDA_WAVE;
+        const dim3 b1(RANK1_NT);
+        if (nv == 0) {
+            hipLaunchKernelGGL(rank1_kernel<0>, dim3(1), b1, 0, s, *a);
+        } else if (nv <= 2) {
+            hipLaunchKernelGGL(rank1_kernel<2>, dim3(1), b1, 0, s, *a);
+        } else if (nv <= 4) {
+            hipLaunchKernelGGL(rank1_kernel<4>, dim3(1), b1, 0, s, *a);
+        } else {
+            hipLaunchKernelGGL((rank1_kernel<RMDA_MAX_EXPERTS / RMDA_WAVE>), dim3(1), b1, 0, s, *a);
+        }
+        return hipGetLastError();
     }
     // one block (up to 1024 pairs): 256 threads; several blocks: 1024, one
     // thread per pair, so each block ranks its pairs in one pass and spreads
