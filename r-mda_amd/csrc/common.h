@@ -64,20 +64,22 @@ __device__ __forceinline__ void rmda_comb_acc8(float acc[8], float w, uint4 q) {
 
 // The hyper-connection update of one token's 8 columns in one stream:
 // h[c + v] += acc[v] * gate (gate = 2 * sigmoid(inj / hc)), h 16-byte aligned.
+__device__ __forceinline__ void rmda_hc_fma8(float4 (&h)[2], const float acc[8], float gate) {
+    h[0].x = __builtin_fmaf(acc[0], gate, h[0].x);
+    h[0].y = __builtin_fmaf(acc[1], gate, h[0].y);
+    h[0].z = __builtin_fmaf(acc[2], gate, h[0].z);
+    h[0].w = __builtin_fmaf(acc[3], gate, h[0].w);
+    h[1].x = __builtin_fmaf(acc[4], gate, h[1].x);
+    h[1].y = __builtin_fmaf(acc[5], gate, h[1].y);
+    h[1].z = __builtin_fmaf(acc[6], gate, h[1].z);
+    h[1].w = __builtin_fmaf(acc[7], gate, h[1].w);
+}
 __device__ __forceinline__ void rmda_hc_acc8(float *h, const float acc[8], float gate) {
     float4 *hp = reinterpret_cast<float4 *>(h);
-    float4 a = hp[0];
-    float4 b = hp[1];
-    a.x = __builtin_fmaf(acc[0], gate, a.x);
-    a.y = __builtin_fmaf(acc[1], gate, a.y);
-    a.z = __builtin_fmaf(acc[2], gate, a.z);
-    a.w = __builtin_fmaf(acc[3], gate, a.w);
-    b.x = __builtin_fmaf(acc[4], gate, b.x);
-    b.y = __builtin_fmaf(acc[5], gate, b.y);
-    b.z = __builtin_fmaf(acc[6], gate, b.z);
-    b.w = __builtin_fmaf(acc[7], gate, b.w);
-    hp[0] = a;
-    hp[1] = b;
+    float4 v[2] = {hp[0], hp[1]};
+    rmda_hc_fma8(v, acc, gate);
+    hp[0] = v[0];
+    hp[1] = v[1];
 }
 
 __device__ __forceinline__ uint4 rmda_pack8_f16(const float acc[8]) {
