@@ -1083,12 +1083,14 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // src/qwen.c:517-539, :844); the second launch also clears gate_up's
     // partial absmax words
     if (rc == RMDA_OK && x32) {
-        rc = hip_check(ctx, rmda_launch_x_absmax(s, args->x32, (size_t)T * d, at<uint32_t>(ws, p.xpart)),
-                       "layer x absmax");
+        uint32_t *part = (size_t)T * d <= RMDA_XCAST1_MAX ? nullptr : at<uint32_t>(ws, p.xpart);
+        if (part != nullptr) {
+            rc = hip_check(ctx, rmda_launch_x_absmax(s, args->x32, (size_t)T * d, part), "layer x absmax");
+        }
         if (rc == RMDA_OK) {
             rc = hip_check(ctx,
-                           rmda_launch_x_cast(s, args->x32, (size_t)T * d, at<uint32_t>(ws, p.xpart),
-                                              at<uint16_t>(ws, p.xs16), xslot, at<uint32_t>(ws, p.hparts)),
+                           rmda_launch_x_cast(s, args->x32, (size_t)T * d, part, at<uint16_t>(ws, p.xs16), xslot,
+                                              at<uint32_t>(ws, p.hparts)),
                            "layer x cast");
         }
     }
@@ -1219,6 +1221,11 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     } else if (rc == RMDA_OK) {
         prof_skip(ctx, RMDA_STAGE_PERMUTE);
     }
+    // x32: the fp32 SwiGLU output.  The strip kernel can cast it as it reads
+    // it, with no pass of its own, where the last region holds it beside the
+    // fp16 expert rows (2 * inter <= d).
+    const bool cast_in_down = x32 && strip_dn && 2 * I <= d && rmda_gemm_strip_casts(items_max, d);
+    float *const hp32 = x32 ? at<float>(ws, p.ye + (cast_in_down ? (size_t)p.groups_rows * d * 2 : 0)) : nullptr;
     rmda_gemm_args_t g{};
     g.items = at<uint32_t>(ws, p.items);
     g.n_items = at<uint32_t>(ws, p.n_items);
@@ -1232,7 +1239,7 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
         g.mode = RMDA_GEMM_SWIGLU;
         g.a = xin;
         g.xscale = xslot;
-        g.hp32 = x32 ? at<float>(ws, p.ye) : nullptr;  // fp32 SwiGLU output, cast below
+        g.hp32 = x32 ? hp32 : nullptr;  // cast below, or by down
         g.hp_amax = x32 ? at<uint32_t>(ws, p.hparts) : nullptr;
         g.rowtok = rowtok;
         g.a_rows = T;
@@ -1261,11 +1268,11 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
                                   "layer gate_up");
     }
     // x32: hp's slot-scaled fp16 cast (src/qwen.c:858-877), routed and shared rows
-    if (rc == RMDA_OK && x32) {
+    if (rc == RMDA_OK && x32 && !cast_in_down) {
         rc = hip_check(ctx,
-                       rmda_launch_hp_cast(s, at<float>(ws, p.ye), hp, at<uint32_t>(ws, p.hparts), hslot,
+                       rmda_launch_hp_cast(s, hp32, hp, at<uint32_t>(ws, p.hparts), hslot,
                                            at<uint32_t>(ws, p.off), at<uint32_t>(ws, p.count), E, I, p.sh_row0,
-                                           p.sh_rows),
+                                           p.sh_rows, p.npairs),
                        "layer hp cast");
     }
     if (rc == RMDA_OK) {
@@ -1283,6 +1290,11 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
         // fp32 rows (the reference's ye) for HF-layout weights, which carry
         // no bound
         g.yscale = hslot;
+        if (cast_in_down) {
+            g.a32 = hp32;
+            g.a_parts = at<uint32_t>(ws, p.hparts);
+            g.a_slot = hslot;
+        }
         g.ye32 = x32 && packed == nullptr ? at<float>(ws, p.ye) : nullptr;
         g.ye_bound = x32 && packed != nullptr ? ye_bound : nullptr;
         // experts averaging 64 rows or more: either tile writes its fp16

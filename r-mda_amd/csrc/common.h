@@ -150,6 +150,15 @@ __device__ __forceinline__ float rmda_slot_inv(const uint32_t *amax) {
     return ldexpf(1.0f, (int)((u >> 23) & 0xffu) - 141);
 }
 
+// the cast_f16.comp scale of an absmax word
+__device__ __forceinline__ float rmda_amax_scale(uint32_t u) {
+    const float a = __builtin_bit_cast(float, u);
+    if (!(a > 0.0f) || __builtin_isinf(a)) {
+        return 1.0f;
+    }
+    return ldexpf(1.0f, 141 - (int)((u >> 23) & 0xffu));
+}
+
 // The slot-scaled mode's fp16 expert rows (packed weights).  bound is the
 // down weights' largest row sum of |w| (rows whose sum is not finite left
 // out), written when the weights are packed.  A SwiGLU output cast with its
@@ -528,6 +537,12 @@ struct rmda_gemm_args_t {
     const uint32_t *yscale;
     float *ye32;
     const uint32_t *ye_bound;
+    // Strip kernel, F16: with a32 set, A is the fp32 SwiGLU output (same
+    // blocked index) and is cast on the way with the slot of the partial
+    // absmax words a_parts, whose fold goes to *a_slot.
+    const float *a32;
+    const uint32_t *a_parts;
+    uint32_t *a_slot;
     // F16, fp16 rows, packed weights: non-zero asks for non-temporal row
     // stores (both tiles' default configurations)
     uint32_t ye_nt;
@@ -588,6 +603,9 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
 // lda, and for F16 the sorted rows * lda, below 2^32 elements.
 // rmda_gemm_strip_pays: the rule for npairs routed rows over `groups` experts
 // (shared one included).
+// rmda_gemm_strip_casts: whether down should cast the fp32 SwiGLU output
+// itself (a32).
+bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w);
 bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k);
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows);
 // Packed slab height: weight rows of one N tile (256 of gate_up's 2 * inter,
@@ -669,6 +687,9 @@ hipError_t rmda_launch_fill_normal(hipStream_t s, void *dst, size_t n, int f16, 
 // absmax to *x_slot and zeroes the RMDA_AMAX_PARTS partial words at
 // hp_parts.  n % 4 == 0, x and x16 16-byte aligned.
 #define RMDA_XCAST_PARTS 256u
+// Up to RMDA_XCAST1_MAX values the cast alone does both: part NULL, every
+// block finds the absmax of all of x itself.
+#define RMDA_XCAST1_MAX 49152u
 hipError_t rmda_launch_x_absmax(hipStream_t s, const float *x, size_t n, uint32_t *part);
 hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uint32_t *part, uint16_t *x16,
                               uint32_t *x_slot, uint32_t *hp_parts);
@@ -679,4 +700,4 @@ hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uin
 // at hp_parts, which block 0 also stores to *slot for the down GEMM.
 hipError_t rmda_launch_hp_cast(hipStream_t s, const float *hp32, uint16_t *hp16, const uint32_t *hp_parts,
                                uint32_t *slot, const uint32_t *off, const uint32_t *count, uint32_t experts,
-                               uint32_t inter, uint32_t sh_row0, uint32_t sh_rows);
+                               uint32_t inter, uint32_t sh_row0, uint32_t sh_rows, uint32_t npairs);

@@ -5,6 +5,8 @@
 //   cast_kernel    shader/cast_f16.comp:20-35 (power-of-two slot scale, RNE)
 //   bf16_kernel    shader/qwen_bf16.comp:9-15 (two bf16 -> two fp16 in place)
 //   fill_kernel    counter hash -> standardised Irwin-Hall(4) -> fp16/fp32
+#include <algorithm>
+
 #include "common.h"
 
 namespace {
@@ -479,15 +481,6 @@ __device__ __forceinline__ uint32_t block_max_bits(float m) {
     return __builtin_bit_cast(uint32_t, red[0]);
 }
 
-// the cast_f16.comp scale of an absmax value (cast_scale without the slot)
-__device__ __forceinline__ float amax_scale(uint32_t u) {
-    const float a = __builtin_bit_cast(float, u);
-    if (!(a > 0.0f) || __builtin_isinf(a)) {
-        return 1.0f;
-    }
-    return ldexpf(1.0f, 141 - (int)((u >> 23) & 0xffu));
-}
-
 __device__ __forceinline__ uint2 cast4(const float4 &v, float sc) {
     return make_uint2((uint32_t)rmda_f2h(v.x * sc) | ((uint32_t)rmda_f2h(v.y * sc) << 16),
                       (uint32_t)rmda_f2h(v.z * sc) | ((uint32_t)rmda_f2h(v.w * sc) << 16));
@@ -553,7 +546,7 @@ __global__ __launch_bounds__(256) void x_cast_kernel(const float4 *__restrict__ 
             hp_parts[threadIdx.x * RMDA_AMAX_STRIDE] = 0u;
         }
     }
-    const float sc = amax_scale(amax);
+    const float sc = rmda_amax_scale(amax);
     constexpr uint32_t U = 4;
     const size_t st = (size_t)gridDim.x * 256;
     size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -570,6 +563,53 @@ __global__ __launch_bounds__(256) void x_cast_kernel(const float4 *__restrict__ 
     }
     for (; i < n4; i += st) {
         x16[i] = cast4(x[i], sc);
+    }
+}
+
+// x_absmax and x_cast in one launch for few values: every block reads all of
+// x (from L2 after the first) for the absmax and casts its own share, in
+// place of a second launch.  Both and the router, MI355X: 1 token of hidden
+// 768 8.7 -> 6.1 us, 4 tokens of hidden 2560 11.2 -> 8.7 us, 16 tokens 12.4 ->
+// 10.5 us, 25 tokens 11.9 -> 12.3 us, hence the bound.
+constexpr uint32_t XC1_NT = 1024;
+constexpr uint32_t XC1_PER = RMDA_XCAST1_MAX / 4 / XC1_NT;  // float4 per thread, at most
+
+__global__ __launch_bounds__(XC1_NT) void x_cast1_kernel(const float4 *__restrict__ x, uint32_t n4,
+                                                         uint2 *__restrict__ x16, uint32_t *__restrict__ x_slot,
+                                                         uint32_t *__restrict__ hp_parts) {
+    __shared__ uint32_t red[XC1_NT / RMDA_WAVE];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t mine = blockIdx.x * XC1_NT + tid;
+    float4 v[XC1_PER];
+#pragma unroll
+    for (uint32_t u = 0; u < XC1_PER; u += 1) {
+        const uint32_t i = tid + u * XC1_NT;
+        v[u] = i < n4 ? x[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    const float4 own = mine < n4 ? x[mine] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (blockIdx.x == 0 && tid < RMDA_AMAX_PARTS) {
+        hp_parts[tid * RMDA_AMAX_STRIDE] = 0u;
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < XC1_PER; u += 1) {
+        m = fmaxf(fmaxf(m, fabsf(v[u].x)), fmaxf(fmaxf(fabsf(v[u].y), fabsf(v[u].z)), fabsf(v[u].w)));
+    }
+    const uint32_t w = rmda_wave_red_u32<true>(__builtin_bit_cast(uint32_t, m));
+    if (tid % RMDA_WAVE == 0) {
+        red[tid / RMDA_WAVE] = w;
+    }
+    __syncthreads();
+    uint32_t amax = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < XC1_NT / RMDA_WAVE; i += 1) {
+        amax = max(amax, red[i]);
+    }
+    if (mine == 0) {
+        *x_slot = amax;
+    }
+    if (mine < n4) {
+        x16[mine] = cast4(own, rmda_amax_scale(amax));
     }
 }
 
@@ -597,7 +637,7 @@ __global__ __launch_bounds__(256) void hp_cast_kernel(const float4 *__restrict__
     const size_t n_r = (size_t)routed_end * inter / 4;
     const size_t s0 = (size_t)sh_row0 * inter / 4;
     const size_t n_s = (size_t)((sh_rows + 15u) / 16u * 16u) * inter / 4;
-    const float sc = amax_scale(s_amax);
+    const float sc = rmda_amax_scale(s_amax);
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n_r + n_s; i += (size_t)gridDim.x * 256) {
         const size_t j = i < n_r ? i : s0 + (i - n_r);
         hp16[j] = cast4(hp32[j], sc);
@@ -614,6 +654,15 @@ hipError_t rmda_launch_x_absmax(hipStream_t s, const float *x, size_t n, uint32_
 
 hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uint32_t *part, uint16_t *x16,
                               uint32_t *x_slot, uint32_t *hp_parts) {
+    if (part == nullptr) {
+        if (n > RMDA_XCAST1_MAX) {
+            return hipErrorInvalidValue;
+        }
+        const uint32_t n4 = (uint32_t)(n / 4);
+        hipLaunchKernelGGL(x_cast1_kernel, dim3((n4 + XC1_NT - 1) / XC1_NT), dim3(XC1_NT), 0, s,
+                           reinterpret_cast<const float4 *>(x), n4, reinterpret_cast<uint2 *>(x16), x_slot, hp_parts);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(x_cast_kernel, dim3(RMDA_XCAST_PARTS), dim3(256), 0, s, reinterpret_cast<const float4 *>(x),
                        n / 4, part, reinterpret_cast<uint2 *>(x16), x_slot, hp_parts);
     return hipGetLastError();
@@ -621,8 +670,11 @@ hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uin
 
 hipError_t rmda_launch_hp_cast(hipStream_t s, const float *hp32, uint16_t *hp16, const uint32_t *hp_parts,
                                uint32_t *slot, const uint32_t *off, const uint32_t *count, uint32_t experts,
-                               uint32_t inter, uint32_t sh_row0, uint32_t sh_rows) {
-    hipLaunchKernelGGL(hp_cast_kernel, dim3(1024), dim3(256), 0, s, reinterpret_cast<const float4 *>(hp32),
+                               uint32_t inter, uint32_t sh_row0, uint32_t sh_rows, uint32_t npairs) {
+    // one thread per four values of the most rows npairs can take up, at most 1024 blocks
+    const uint64_t rows = (uint64_t)npairs + 15ull * std::min(npairs, experts) + sh_rows + 15u;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(1024, (rows * inter / 4 + 255) / 256);
+    hipLaunchKernelGGL(hp_cast_kernel, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float4 *>(hp32),
                        reinterpret_cast<uint2 *>(hp16), hp_parts, slot, off, count, experts, inter, sh_row0,
                        sh_rows);
     return hipGetLastError();

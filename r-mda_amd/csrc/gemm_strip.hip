@@ -43,10 +43,38 @@ constexpr uint32_t STEP = SLAB * BK;
 constexpr uint32_t STRIPS = 8;     // strips of 32 weight rows in a slab
 constexpr uint32_t CHUNK = 64;     // rows of a chunk
 
+typedef float float8_t __attribute__((ext_vector_type(8)));
+
+// One MFMA operand of A as it is loaded: fp16, or (CAST) fp32 to be scaled
+// and rounded as hp_cast_kernel does it.
+template <bool CAST>
+struct a_frag_t {
+    half8_t v;
+    __device__ __forceinline__ void load(const rmda_gemm_args_t &g, uint32_t i) {
+        v = *reinterpret_cast<const half8_t *>(g.a + i);
+    }
+    __device__ __forceinline__ half8_t get(float) const { return v; }
+};
+template <>
+struct a_frag_t<true> {
+    float8_t v;
+    __device__ __forceinline__ void load(const rmda_gemm_args_t &g, uint32_t i) {
+        v = *reinterpret_cast<const float8_t *>(g.a32 + i);
+    }
+    __device__ __forceinline__ half8_t get(float scale) const {
+        half8_t h;
+#pragma unroll
+        for (int j = 0; j < 8; j += 1) {
+            h[j] = (_Float16)(v[j] * scale);
+        }
+        return h;
+    }
+};
+
 // One chunk of MT live 16-row groups times one strip.
-template <int MODE, int MT, int DEPTH, bool SC>
+template <int MODE, int MT, int DEPTH, bool SC, bool CAST>
 __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t row0, uint32_t rows, bool is_shared,
-                                            const uint16_t *b0, const uint16_t *b1, uint32_t col0) {
+                                            const uint16_t *b0, const uint16_t *b1, uint32_t col0, float scale) {
     const uint32_t lane = threadIdx.x;
     const uint32_t fr = lane % 16;
     const uint32_t fq = lane / 16;
@@ -65,7 +93,8 @@ __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t 
             a[m] = (uint32_t)rmda_hp_index(row0 + (uint32_t)m * 16u, 0, g.lda) + fr * 32 + fq * 8;
         }
     }
-    half8_t ra[DEPTH][MT], rb[DEPTH][2];
+    a_frag_t<CAST> ra[DEPTH][MT];
+    half8_t rb[DEPTH][2];
     floatx4_t acc[MT][2];
 #pragma unroll
     for (int m = 0; m < MT; m += 1) {
@@ -77,14 +106,15 @@ __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t 
         rb[u][1] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(b1 + (size_t)s * STEP));
 #pragma unroll
         for (int m = 0; m < MT; m += 1) {
-            ra[u][m] = *reinterpret_cast<const half8_t *>(g.a + s * A_STEP + a[m]);
+            ra[u][m].load(g, s * A_STEP + a[m]);
         }
     };
     auto mma = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
         for (int m = 0; m < MT; m += 1) {
-            acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra[u][m], rb[u][0], acc[m][0], 0, 0, 0);
-            acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra[u][m], rb[u][1], acc[m][1], 0, 0, 0);
+            const half8_t av = ra[u][m].get(scale);
+            acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, rb[u][0], acc[m][0], 0, 0, 0);
+            acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, rb[u][1], acc[m][1], 0, 0, 0);
         }
     };
 #pragma unroll
@@ -150,10 +180,19 @@ __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t 
 // the shallow ring covers at once only pays for its longer start (one token:
 // 36.1 -> 37.3 us), and a K loop shorter than the ring reads its last step
 // again (K = 256: down 15.7 -> 21.0 us).
-template <int MODE, bool DEEP, bool SC>
+template <int MODE, bool DEEP, bool SC, bool CAST>
 __global__ __launch_bounds__(RMDA_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) void strip_kernel(
     rmda_gemm_args_t g, uint32_t chunks) {
     const const_u32p items = (const_u32p)g.items;
+    float scale = 1.0f;
+    if constexpr (CAST) {
+        static_assert(RMDA_AMAX_PARTS == RMDA_WAVE, "one partial word per lane");
+        const uint32_t m = rmda_wave_red_u32<true>(g.a_parts[threadIdx.x * RMDA_AMAX_STRIDE]);
+        scale = rmda_amax_scale(m);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            *g.a_slot = m;  // for the combine
+        }
+    }
     // blockIdx.x = (slab / 8, chunk, strip, slab % 8), slabs counted over the
     // whole work list: the strips and row chunks of a slab share an XCD's L2
     const uint32_t nslab = g.n_w / SLAB;
@@ -186,10 +225,10 @@ __global__ __launch_bounds__(RMDA_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2)
         wg + (size_t)slab * (g.k / BK) * STEP + nb * BK + fr * BK + (fq ^ swz<BK>(fr)) * 8;
     const uint16_t *const b1 = b0 + (MODE == RMDA_GEMM_SWIGLU ? 32u : 16u) * BK;
     switch ((rows + 15u) / 16u) {
-    case 1: strip_chunk<MODE, 1, DEEP ? 16 : 8, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
-    case 2: strip_chunk<MODE, 2, DEEP ? 12 : 8, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
-    case 3: strip_chunk<MODE, 3, DEEP ? 8 : 6, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
-    default: strip_chunk<MODE, 4, DEEP ? 7 : 6, SC>(g, row0, rows, is_shared, b0, b1, col0); break;
+    case 1: strip_chunk<MODE, 1, DEEP ? 16 : 8, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
+    case 2: strip_chunk<MODE, 2, DEEP ? 12 : 8, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
+    case 3: strip_chunk<MODE, 3, DEEP ? 8 : 6, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
+    default: strip_chunk<MODE, 4, DEEP ? 7 : CAST ? 5 : 6, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
     }
 }
 
@@ -198,10 +237,16 @@ hipError_t launch_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items
     const uint32_t chunks = (item_rows + CHUNK - 1) / CHUNK;
     const dim3 grid((items * (a->n_w / SLAB) + 7) / 8 * 8 * STRIPS * chunks);
     const bool sc = a->hp32 != nullptr || a->ye_bound != nullptr;
+    if constexpr (MODE == RMDA_GEMM_F16 && !DEEP) {
+        if (a->a32 != nullptr) {
+            hipLaunchKernelGGL((strip_kernel<MODE, false, true, true>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+            return hipGetLastError();
+        }
+    }
     if (sc) {
-        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, true>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, true, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
     } else {
-        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, false, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
     }
     return hipGetLastError();
 }
@@ -228,8 +273,17 @@ bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint
     return tasks <= 256 && bytes * ((uint64_t)npairs + 32ull * groups) / (64ull * groups) <= (64ull << 20);
 }
 
+bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w) {
+    // Casting in down spares a launch, but every strip converts the rows
+    // again and reads twice the bytes: hp cast + down, 24 waves of hidden 768,
+    // width 256 7.0 -> 4.2 us; 336 waves of hidden 512, width 384 10.9 -> 9.4;
+    // 880 waves of hidden 2560, width 640 21.5 -> 21.9; 11000 waves 224 -> 239.
+    return (uint64_t)items * (n_w / 32u) <= 512;
+}
+
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
-    if (a->n_w % SLAB != 0 || a->k % BK != 0 || a->n_items == nullptr || a->fc.cnt != nullptr || a->ye32 != nullptr) {
+    if (a->n_w % SLAB != 0 || a->k % BK != 0 || a->n_items == nullptr || a->fc.cnt != nullptr || a->ye32 != nullptr ||
+        (a->a32 != nullptr && (a->mode != RMDA_GEMM_F16 || a->ye_bound == nullptr))) {
         return hipErrorInvalidValue;
     }
     if (items == 0 || item_rows == 0) {
@@ -237,7 +291,7 @@ hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint
     }
     // more waves than the chip holds at once (two per SIMD), and a K loop that
     // fills the deep ring
-    const bool deep = (uint64_t)items * (a->n_w / 32u) > 2048 && a->k >= 16 * BK;
+    const bool deep = (uint64_t)items * (a->n_w / 32u) > 2048 && a->k >= 16 * BK && a->a32 == nullptr;
     if (a->mode == RMDA_GEMM_SWIGLU) {
         return deep ? launch_strip<RMDA_GEMM_SWIGLU, true>(s, a, items, item_rows)
                     : launch_strip<RMDA_GEMM_SWIGLU, false>(s, a, items, item_rows);
