@@ -1088,9 +1088,13 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
             rc = hip_check(ctx, rmda_launch_x_absmax(s, args->x32, (size_t)T * d, part), "layer x absmax");
         }
         if (rc == RMDA_OK) {
+            rmda_xcast_more_t more{};
+            more.zero = at<uint32_t>(ws, p.hparts);
+            more.n_zero = RMDA_AMAX_PARTS;
+            more.zero_stride = RMDA_AMAX_STRIDE;
             rc = hip_check(ctx,
                            rmda_launch_x_cast(s, args->x32, (size_t)T * d, part, at<uint16_t>(ws, p.xs16), xslot,
-                                              at<uint32_t>(ws, p.hparts)),
+                                              &more),
                            "layer x cast");
         }
     }
@@ -1842,22 +1846,6 @@ uint32_t shim_slot(rmda_qwen_moe_t *q) {
     return q->n_slots++;
 }
 
-// mda_qwen_cast (src/qwen.c:517-539): absmax into a new slot, then the cast
-int shim_cast(rmda_qwen_moe_t *q, const ShimPlan &p, const float *src, uint16_t *dst, uint32_t n, uint32_t *slot) {
-    *slot = shim_slot(q);
-    if (*slot == RMDA_NO_SLOT) {
-        return q->ctx->err;
-    }
-    uint32_t *amax = scr<uint32_t>(q, p.amax);
-    const rmda_pc_absmax_t pa{n, *slot};
-    int rc = rmda_absmax(q->ctx, &pa, src, amax);
-    if (rc == RMDA_OK) {
-        const rmda_pc_cast_t pc{n, *slot};
-        rc = rmda_cast_f16(q->ctx, &pc, src, dst, amax);
-    }
-    return rc;
-}
-
 }  // namespace
 
 size_t rmda_qwen_moe_scratch_bytes(const rmda_qwen_moe_t *q) {
@@ -1938,13 +1926,27 @@ int route_rec(rmda_qwen_moe_t *q, uint32_t rows, uint32_t mrows, bool zero_xp) {
             return rc;
         }
     }
-    const rmda_pc_moe_route_t pr{rows, q->experts, q->topk, p.ps};
-    rc = rmda_moe_route(q->ctx, &pr, scr<float>(q, p.p), scr<uint32_t>(q, p.idx), scr<float>(q, p.wt),
-                        scr<uint32_t>(q, p.count));
-    if (rc == RMDA_OK) {
-        const rmda_pc_moe_scan_t ps{q->experts, RMDA_QWEN_TILE};
-        rc = rmda_moe_scan(q->ctx, &ps, scr<uint32_t>(q, p.count), scr<uint32_t>(q, p.off),
-                           scr<uint32_t>(q, p.tiles), mrows / RMDA_QWEN_TILE);
+    const uint32_t npairs = rows * q->topk;  // <= RMDA_CTX_MAX_PAIRS (shim_ok)
+    uint32_t *idx = scr<uint32_t>(q, p.idx), *count = scr<uint32_t>(q, p.count), *off = scr<uint32_t>(q, p.off);
+    if (npairs <= RMDA_COUNT1_MAX_PAIRS) {
+        // rmda_moe_route and rmda_moe_scan with the counts and offsets in one launch
+        rc = hip_check(q->ctx,
+                       rmda_launch_route(q->ctx->stream, scr<float>(q, p.p), idx, scr<float>(q, p.wt), nullptr, rows,
+                                         q->experts, q->topk, p.ps),
+                       "route_rec route");
+        if (rc == RMDA_OK) {
+            rc = hip_check(q->ctx,
+                           rmda_launch_count_scan(q->ctx->stream, idx, npairs, q->experts, count, off,
+                                                  scr<uint32_t>(q, p.tiles), mrows / RMDA_QWEN_TILE, RMDA_QWEN_TILE),
+                           "route_rec scan");
+        }
+    } else {
+        const rmda_pc_moe_route_t pr{rows, q->experts, q->topk, p.ps};
+        rc = rmda_moe_route(q->ctx, &pr, scr<float>(q, p.p), idx, scr<float>(q, p.wt), count);
+        if (rc == RMDA_OK) {
+            const rmda_pc_moe_scan_t ps{q->experts, RMDA_QWEN_TILE};
+            rc = rmda_moe_scan(q->ctx, &ps, count, off, scr<uint32_t>(q, p.tiles), mrows / RMDA_QWEN_TILE);
+        }
     }
     if (rc == RMDA_OK) {
         rc = rmda_moe_scatter_experts(q->ctx, q->experts);
@@ -1985,25 +1987,66 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
     const uint32_t mrows = qwen_moe_rows(rows, K, E);
     const uint32_t rows_pad = (rows + RMDA_QWEN_TILE - 1) / RMDA_QWEN_TILE * RMDA_QWEN_TILE;
     uint32_t *amax = scr<uint32_t>(q, p.amax);
-    // mda_qwen_slots_begin (src/qwen.c:500-503)
+    // mda_qwen_slots_begin (src/qwen.c:500-503), A0: x cast with a slot
+    // (src/qwen.c:844); the fp32 router reads the same cast and multiplies
+    // each chunk sum by the slot's inverse scale, which for fp16-range
+    // activations gives the logits of x itself bit for bit and keeps
+    // activations outside that range (subnormal or above 65504 as fp16) at
+    // full precision.  The router matrix is repacked into the order the router
+    // kernel streams (the HF-layout kernel takes about three times as long),
+    // the same logits bit for bit.  The cast's launch also clears the other
+    // slots, packs the router and writes the shared expert's tile map and
+    // segment, four launches less than one by one.
     q->n_slots = 0;
-    rc = hip_check(c, rmda_launch_zero(c->stream, amax, RMDA_QWEN_MAX_SLOTS, 0), "moe_rec slot fill");
-    // A0: x cast with a slot (src/qwen.c:844); the fp32 router reads the same
-    // cast and multiplies each chunk sum by the slot's inverse scale, which
-    // for fp16-range activations gives the logits of x itself bit for bit
-    // and keeps activations outside that range (subnormal or above 65504 as
-    // fp16) at full precision
-    uint32_t sx = RMDA_NO_SLOT;
-    if (rc == RMDA_OK) {
-        rc = shim_cast(q, p, x, scr<uint16_t>(q, p.a16), rows * d, &sx);
-    }
-    // the router projection on the router matrix repacked into the order the
-    // router kernel streams (3.6 us for 128 x 2048 at config 3; the HF-layout
-    // kernel takes about three times as long as the packed one), the same
-    // logits bit for bit
-    if (rc == RMDA_OK) {
-        rc = hip_check(c, rmda_launch_router_pack(c->stream, q->w_router, scr<float>(q, p.wr), p.ps, d),
-                       "moe_rec router pack");
+    const uint32_t sx = shim_slot(q);
+    uint32_t *const tiles1 = S > 0 ? scr<uint32_t>(q, p.tiles1) : nullptr;
+    uint32_t *const live1 = amax + RMDA_QWEN_MAX_SLOTS;  // {0, rows}: the words behind the slots
+    if (aligned(x, 16)) {
+        rmda_xcast_more_t more{};
+        more.zero = amax;
+        more.n_zero = RMDA_QWEN_MAX_SLOTS;
+        more.zero_stride = 1;
+        more.w_router = q->w_router;
+        more.router = scr<float>(q, p.wr);
+        more.router_cols = p.ps;
+        more.d = d;
+        more.tiles1 = tiles1;
+        more.n_tiles1 = rows_pad / RMDA_QWEN_TILE;
+        more.live1 = live1;
+        more.rows = rows;
+        const size_t n = (size_t)rows * d;
+        // the partial maxima lie in xp, which the scatter below fills
+        uint32_t *part = n <= RMDA_XCAST1_MAX ? nullptr : scr<uint32_t>(q, p.xp);
+        if (part != nullptr) {
+            rc = hip_check(c, rmda_launch_x_absmax(c->stream, x, n, part), "moe_rec x absmax");
+        }
+        if (rc == RMDA_OK) {
+            rc = hip_check(c, rmda_launch_x_cast(c->stream, x, n, part, scr<uint16_t>(q, p.a16), amax + sx, &more),
+                           "moe_rec x cast");
+        }
+    } else {
+        rc = hip_check(c, rmda_launch_zero(c->stream, amax, RMDA_QWEN_MAX_SLOTS, 0), "moe_rec slot fill");
+        const rmda_pc_absmax_t pa{rows * d, sx};
+        if (rc == RMDA_OK) {
+            rc = rmda_absmax(c, &pa, x, amax);
+        }
+        const rmda_pc_cast_t pc{rows * d, sx};
+        if (rc == RMDA_OK) {
+            rc = rmda_cast_f16(c, &pc, x, scr<uint16_t>(q, p.a16), amax);
+        }
+        if (rc == RMDA_OK) {
+            rc = hip_check(c, rmda_launch_router_pack(c->stream, q->w_router, scr<float>(q, p.wr), p.ps, d),
+                           "moe_rec router pack");
+        }
+        if (rc == RMDA_OK && S > 0) {
+            rc = hip_check(c, rmda_launch_zero(c->stream, tiles1, rows_pad / RMDA_QWEN_TILE, 0), "moe_rec shared tiles");
+        }
+        if (rc == RMDA_OK && S > 0) {
+            rc = hip_check(c, rmda_launch_zero(c->stream, live1, 1, 0), "moe_rec shared segment");
+        }
+        if (rc == RMDA_OK && S > 0) {
+            rc = hip_check(c, rmda_launch_zero(c->stream, live1 + 1, 1, rows), "moe_rec shared segment");
+        }
     }
     if (rc == RMDA_OK) {
         rc = hip_check(c,
@@ -2057,20 +2100,18 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
     // A8: the shared expert as one-expert grouped GEMMs over the padded rows
     // (src/qwen.c:879-886); rows past `rows` hold stale data and are unused
     if (rc == RMDA_OK && S > 0) {
-        uint32_t *t1 = scr<uint32_t>(q, p.tiles1);
-        rc = hip_check(c, rmda_launch_zero(c->stream, t1, rows_pad / RMDA_QWEN_TILE, 0), "moe_rec shared tiles");
+        // gate_up with SwiGLU and its absmax in the epilogue, then the scaled
+        // cast, as for the routed experts above; live1 keeps the padding rows
+        // out of the absmax
+        const uint32_t ss = shim_slot(q);
+        rc = ss == RMDA_NO_SLOT ? c->err : RMDA_OK;
+        mm_swiglu_t ssw{scr<float>(q, p.hs), ss, false};
         if (rc == RMDA_OK) {
             const rmda_pc_moe_mm_t pm{rows_pad, 2 * S, d, sx, RMDA_NO_SLOT};
-            rc = rmda_moe_mm(c, &pm, scr<uint16_t>(q, p.a16), q->w_sh_gate_up, scr<float>(q, p.gs), amax, t1);
+            rc = moe_mm(c, &pm, scr<uint16_t>(q, p.a16), q->w_sh_gate_up, scr<float>(q, p.gs), amax, tiles1, live1,
+                        live1 + 1, &ssw);
         }
-        // SwiGLU with the absmax of hs folded in, then the scaled cast (as
-        // for the routed experts above)
-        uint32_t ss = RMDA_NO_SLOT;
-        if (rc == RMDA_OK) {
-            ss = shim_slot(q);
-            rc = ss == RMDA_NO_SLOT ? c->err : RMDA_OK;
-        }
-        if (rc == RMDA_OK) {
+        if (rc == RMDA_OK && !ssw.fused) {
             const rmda_pc_qwen_elem_t pe{rows, S, 2 * S, 0, S, 0, 1.0f};
             rc = hip_check(c, rmda_launch_elem_absmax(c->stream, &pe, scr<float>(q, p.gs), scr<float>(q, p.hs), amax,
                                                       ss),
@@ -2082,7 +2123,8 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
         }
         if (rc == RMDA_OK) {
             const rmda_pc_moe_mm_t pm{rows_pad, d, S, ss, RMDA_NO_SLOT};
-            rc = rmda_moe_mm(c, &pm, scr<uint16_t>(q, p.hs16), q->w_sh_down, scr<float>(q, p.sh), amax, t1);
+            rc = moe_mm(c, &pm, scr<uint16_t>(q, p.hs16), q->w_sh_down, scr<float>(q, p.sh), amax, tiles1, live1,
+                        live1 + 1);
         }
     }
     // A9: combine (src/qwen.c:887-906)

@@ -337,13 +337,12 @@ hipError_t rmda_launch_router(hipStream_t s, const uint16_t *x16, const float *w
 __host__ __device__ __forceinline__ uint32_t rmda_router_cpad(uint32_t cols) {
     return (cols + RMDA_WAVE - 1) / RMDA_WAVE * RMDA_WAVE;
 }
-// Block b of nb's share of the router packing (256 threads), zero columns
-// past `cols`.
+// Block b of nb's share of the router packing, zero columns past `cols`.
 __device__ __forceinline__ void rmda_router_pack_share(const float *__restrict__ w, float *__restrict__ out,
                                                        uint32_t cols, uint32_t d, uint32_t b, uint32_t nb) {
     const uint32_t cpad = rmda_router_cpad(cols);
     const size_t n = (size_t)d * cpad;
-    for (size_t o = (size_t)b * 256 + threadIdx.x; o < n; o += (size_t)nb * 256) {
+    for (size_t o = (size_t)b * blockDim.x + threadIdx.x; o < n; o += (size_t)nb * blockDim.x) {
         const uint32_t j = (uint32_t)(o % 16);
         const uint32_t c = (uint32_t)((o / 16) % cpad);
         const uint32_t k = (uint32_t)(o / (16 * (size_t)cpad)) * 16 + (j % 4) * 4 + j / 4;
@@ -436,6 +435,9 @@ hipError_t rmda_launch_rank(hipStream_t s, const rmda_rank_args_t *a);
 #define RMDA_COUNT1_MAX_PAIRS (1u << 16)
 hipError_t rmda_launch_count(hipStream_t s, const uint32_t *idx, uint32_t npairs, uint32_t experts,
                              uint32_t *count);
+// scan.hip: rmda_launch_count, then rmda_launch_scan on its counts, in one launch
+hipError_t rmda_launch_count_scan(hipStream_t s, const uint32_t *idx, uint32_t npairs, uint32_t experts,
+                                  uint32_t *count, uint32_t *off, uint32_t *tiles, uint32_t n_tiles, uint32_t tile);
 
 // scatter.hip: slot[pr] = boff[pr/BLOCK][e] + lrank[pr]; optional row copy
 // (xp) and inverse map (rowtok[slot] = token).
@@ -679,20 +681,31 @@ hipError_t rmda_launch_cast(hipStream_t s, const rmda_pc_cast_t *pc, const float
 hipError_t rmda_launch_bf16(hipStream_t s, uint32_t n, uint32_t *w);
 hipError_t rmda_launch_fill_normal(hipStream_t s, void *dst, size_t n, int f16, uint64_t stream,
                                    uint64_t seed, float std);
-// The fused layer's fp32-activation input, in two launches (the reference's
-// absmax.comp + cast_f16.comp with a fresh slot, src/qwen.c:517-539, with no
-// zero-filled slot word needed beforehand): part[b] = the absmax bits of
-// block b's share of x (nparts blocks), then every block folds the parts,
-// casts its share of x with the slot scale into x16, and block 0 stores the
-// absmax to *x_slot and zeroes the RMDA_AMAX_PARTS partial words at
-// hp_parts.  n % 4 == 0, x and x16 16-byte aligned.
+// fp32 activations with a fresh scale slot (the reference's absmax.comp +
+// cast_f16.comp, src/qwen.c:517-539, with no zero-filled slot word needed
+// beforehand), in two launches: part[b] = the absmax bits of block b's share
+// of x (RMDA_XCAST_PARTS blocks), then every block folds the parts, casts its
+// share of x with the slot scale into x16, and block 0 stores the absmax to
+// *x_slot.  Up to RMDA_XCAST1_MAX values the cast alone does both: part NULL,
+// every block finds the absmax of all of x itself.  n % 4 == 0, x and x16
+// 16-byte aligned.  The cast's launch also does what its caller has to have
+// done by then (rmda_xcast_more_t).
 #define RMDA_XCAST_PARTS 256u
-// Up to RMDA_XCAST1_MAX values the cast alone does both: part NULL, every
-// block finds the absmax of all of x itself.
 #define RMDA_XCAST1_MAX 49152u
+struct rmda_xcast_more_t {
+    uint32_t *zero;         // words cleared, n_zero of them zero_stride apart (*x_slot excepted); n_zero <= 256
+    uint32_t n_zero, zero_stride;
+    const float *w_router;  // or NULL: packed into `router` as rmda_launch_router_pack does
+    float *router;
+    uint32_t router_cols, d;
+    uint32_t *tiles1;       // or NULL: the shared expert's tile map, n_tiles1 zeros,
+    uint32_t n_tiles1;      // and its segment live1 = {0, rows}
+    uint32_t *live1;
+    uint32_t rows;
+};
 hipError_t rmda_launch_x_absmax(hipStream_t s, const float *x, size_t n, uint32_t *part);
 hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uint32_t *part, uint16_t *x16,
-                              uint32_t *x_slot, uint32_t *hp_parts);
+                              uint32_t *x_slot, const rmda_xcast_more_t *more);
 // hp16[i] = fp16(hp32[i] * scale(amax)) over the blocked hp of the slot-scaled
 // mode, for the routed rows [0, off[E-1] + count[E-1] rounded up to 16) and,
 // when sh_rows > 0, the shared expert's rows [sh_row0, sh_row0 + sh_rows

@@ -520,11 +520,31 @@ __global__ __launch_bounds__(256) void x_absmax_kernel(const float4 *__restrict_
     }
 }
 
+// block 0's part of rmda_xcast_more_t
+__device__ __forceinline__ void xcast_more(const rmda_xcast_more_t &m, const uint32_t *x_slot) {
+    if (threadIdx.x < m.n_zero && m.zero + threadIdx.x * m.zero_stride != x_slot) {
+        m.zero[threadIdx.x * m.zero_stride] = 0u;
+    }
+    if (m.tiles1 != nullptr) {
+        for (uint32_t i = threadIdx.x; i < m.n_tiles1; i += blockDim.x) {
+            m.tiles1[i] = 0u;
+        }
+        if (threadIdx.x < 2) {
+            m.live1[threadIdx.x] = threadIdx.x == 0 ? 0u : m.rows;
+        }
+    }
+}
+
 // every block folds the parts (the values are non-negative, so their bit
 // patterns order as the values do), then cast_f16.comp over its share
 __global__ __launch_bounds__(256) void x_cast_kernel(const float4 *__restrict__ x, size_t n4,
                                                      const uint32_t *__restrict__ part, uint2 *__restrict__ x16,
-                                                     uint32_t *__restrict__ x_slot, uint32_t *__restrict__ hp_parts) {
+                                                     uint32_t *x_slot, rmda_xcast_more_t more) {
+    if (blockIdx.x >= RMDA_XCAST_PARTS) {
+        rmda_router_pack_share(more.w_router, more.router, more.router_cols, more.d, blockIdx.x - RMDA_XCAST_PARTS,
+                               gridDim.x - RMDA_XCAST_PARTS);
+        return;
+    }
     __shared__ uint32_t s_amax;
     if (threadIdx.x < RMDA_WAVE) {
         uint32_t m = 0;
@@ -542,13 +562,11 @@ __global__ __launch_bounds__(256) void x_cast_kernel(const float4 *__restrict__ 
         if (threadIdx.x == 0) {
             *x_slot = amax;
         }
-        if (threadIdx.x < RMDA_AMAX_PARTS) {
-            hp_parts[threadIdx.x * RMDA_AMAX_STRIDE] = 0u;
-        }
+        xcast_more(more, x_slot);
     }
     const float sc = rmda_amax_scale(amax);
     constexpr uint32_t U = 4;
-    const size_t st = (size_t)gridDim.x * 256;
+    constexpr size_t st = (size_t)RMDA_XCAST_PARTS * 256;
     size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     for (; i + (U - 1) * st < n4; i += U * st) {
         float4 v[U];
@@ -575,8 +593,13 @@ constexpr uint32_t XC1_NT = 1024;
 constexpr uint32_t XC1_PER = RMDA_XCAST1_MAX / 4 / XC1_NT;  // float4 per thread, at most
 
 __global__ __launch_bounds__(XC1_NT) void x_cast1_kernel(const float4 *__restrict__ x, uint32_t n4,
-                                                         uint2 *__restrict__ x16, uint32_t *__restrict__ x_slot,
-                                                         uint32_t *__restrict__ hp_parts) {
+                                                         uint32_t cast_blocks, uint2 *__restrict__ x16,
+                                                         uint32_t *x_slot, rmda_xcast_more_t more) {
+    if (blockIdx.x >= cast_blocks) {
+        rmda_router_pack_share(more.w_router, more.router, more.router_cols, more.d, blockIdx.x - cast_blocks,
+                               gridDim.x - cast_blocks);
+        return;
+    }
     __shared__ uint32_t red[XC1_NT / RMDA_WAVE];
     const uint32_t tid = threadIdx.x;
     const uint32_t mine = blockIdx.x * XC1_NT + tid;
@@ -587,8 +610,8 @@ __global__ __launch_bounds__(XC1_NT) void x_cast1_kernel(const float4 *__restric
         v[u] = i < n4 ? x[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     const float4 own = mine < n4 ? x[mine] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (blockIdx.x == 0 && tid < RMDA_AMAX_PARTS) {
-        hp_parts[tid * RMDA_AMAX_STRIDE] = 0u;
+    if (blockIdx.x == 0) {
+        xcast_more(more, x_slot);
     }
     float m = 0.0f;
 #pragma unroll
@@ -653,18 +676,26 @@ hipError_t rmda_launch_x_absmax(hipStream_t s, const float *x, size_t n, uint32_
 }
 
 hipError_t rmda_launch_x_cast(hipStream_t s, const float *x, size_t n, const uint32_t *part, uint16_t *x16,
-                              uint32_t *x_slot, uint32_t *hp_parts) {
-    if (part == nullptr) {
-        if (n > RMDA_XCAST1_MAX) {
-            return hipErrorInvalidValue;
-        }
-        const uint32_t n4 = (uint32_t)(n / 4);
-        hipLaunchKernelGGL(x_cast1_kernel, dim3((n4 + XC1_NT - 1) / XC1_NT), dim3(XC1_NT), 0, s,
-                           reinterpret_cast<const float4 *>(x), n4, reinterpret_cast<uint2 *>(x16), x_slot, hp_parts);
-        return hipGetLastError();
+                              uint32_t *x_slot, const rmda_xcast_more_t *more) {
+    if (more->n_zero > 256 || (part == nullptr && n > RMDA_XCAST1_MAX)) {
+        return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(x_cast_kernel, dim3(RMDA_XCAST_PARTS), dim3(256), 0, s, reinterpret_cast<const float4 *>(x),
-                       n / 4, part, reinterpret_cast<uint2 *>(x16), x_slot, hp_parts);
+    const uint32_t nt = part == nullptr ? XC1_NT : 256u;
+    uint32_t pack = 0;  // blocks of the router packing
+    if (more->w_router != nullptr) {
+        pack = (uint32_t)std::min<size_t>(((size_t)more->d * rmda_router_cpad(more->router_cols) + nt - 1) / nt,
+                                          1048576u / nt);
+    }
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    uint2 *o4 = reinterpret_cast<uint2 *>(x16);
+    if (part == nullptr) {
+        const uint32_t n4 = (uint32_t)(n / 4);
+        const uint32_t cast = (n4 + XC1_NT - 1) / XC1_NT;
+        hipLaunchKernelGGL(x_cast1_kernel, dim3(cast + pack), dim3(XC1_NT), 0, s, x4, n4, cast, o4, x_slot, *more);
+    } else {
+        hipLaunchKernelGGL(x_cast_kernel, dim3(RMDA_XCAST_PARTS + pack), dim3(256), 0, s, x4, n / 4, part, o4, x_slot,
+                           *more);
+    }
     return hipGetLastError();
 }
 

@@ -96,9 +96,29 @@ __device__ uint32_t block_exscan3(uint32_t v, uint32_t u1, uint32_t u2, uint32_t
     return base + x[0] - v;
 }
 
+// tiles[t] = the expert whose padded rows hold row t * tile, or RMDA_NONE:
+// written once per t, found by binary search over the experts' inclusive
+// padded ends instead of relying on a pre-fill.
+__device__ __forceinline__ void fill_tiles(const uint32_t *end, uint32_t *__restrict__ tiles, uint32_t n_tiles,
+                                           uint32_t experts, uint32_t tile, uint32_t nt) {
+    for (uint32_t t = threadIdx.x; t < n_tiles; t += nt) {
+        // first expert whose inclusive end exceeds t*tile
+        const uint64_t row = (uint64_t)t * tile;
+        uint32_t lo = 0;
+        uint32_t hi = experts;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if ((uint64_t)end[mid] > row) {
+                hi = mid;
+            } else {
+                lo = mid + 1;
+            }
+        }
+        tiles[t] = lo < experts ? lo : RMDA_NONE;
+    }
+}
+
 // shader/moe_scan.comp:14-37, one thread per expert (experts <= 512).
-// tiles[t] is written once per t: the owner is found by binary search over
-// the inclusive padded prefix instead of relying on a pre-fill.
 __global__ __launch_bounds__(512) void scan_kernel(const uint32_t *__restrict__ count,
                                                    uint32_t *__restrict__ off,
                                                    uint32_t *__restrict__ tiles,
@@ -124,21 +144,7 @@ __global__ __launch_bounds__(512) void scan_kernel(const uint32_t *__restrict__ 
     if (e < experts) {
         off[e] = s[e] - p;
     }
-    for (uint32_t t = e; t < n_tiles; t += 512) {
-        // first expert whose inclusive end exceeds t*tile
-        const uint64_t row = (uint64_t)t * tile;
-        uint32_t lo = 0;
-        uint32_t hi = experts;
-        while (lo < hi) {
-            uint32_t mid = (lo + hi) / 2;
-            if ((uint64_t)s[mid] > row) {
-                hi = mid;
-            } else {
-                lo = mid + 1;
-            }
-        }
-        tiles[t] = lo < experts ? lo : RMDA_NONE;
-    }
+    fill_tiles(s, tiles, n_tiles, experts, tile, 512);
 }
 
 // Upper bound on the polls of a rank block that waits for the routing
@@ -780,9 +786,10 @@ __global__ __launch_bounds__(RANK1_NT) void rank1_kernel(rmda_rank_args_t a) {
 // RMDA_COUNT1_MAX_PAIRS pairs: one 1024-thread block, an LDS histogram, no
 // hand-off between blocks.  Four 16-byte loads per thread in flight when idx
 // is 16-byte aligned.
+// s_count: the counts again, in LDS, for a caller that goes on with them.
 template <bool VEC>
-__global__ __launch_bounds__(1024) void count_kernel(const uint32_t *__restrict__ idx, uint32_t npairs,
-                                                     uint32_t experts, uint32_t *__restrict__ count) {
+__device__ __forceinline__ void count_block(const uint32_t *__restrict__ idx, uint32_t npairs, uint32_t experts,
+                                            uint32_t *__restrict__ count, uint32_t *s_count) {
     // CS copies of the histogram, lane l adding to copy l % CS (rows of CW
     // words, one spare so that the copies of one expert sit in different
     // banks): under skewed routing many lanes of a wave hold the same expert,
@@ -834,7 +841,39 @@ __global__ __launch_bounds__(1024) void count_kernel(const uint32_t *__restrict_
             n += hc[c * CW + e];
         }
         count[e] = n;
+        if (s_count != nullptr) {
+            s_count[e] = n;
+        }
     }
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(1024) void count_kernel(const uint32_t *__restrict__ idx, uint32_t npairs,
+                                                     uint32_t experts, uint32_t *__restrict__ count) {
+    count_block<VEC>(idx, npairs, experts, count, nullptr);
+}
+
+// count_kernel, then scan_kernel's offsets and tile map from the counts
+template <bool VEC>
+__global__ __launch_bounds__(1024) void count_scan_kernel(const uint32_t *__restrict__ idx, uint32_t npairs,
+                                                          uint32_t experts, uint32_t *__restrict__ count,
+                                                          uint32_t *__restrict__ off, uint32_t *__restrict__ tiles,
+                                                          uint32_t n_tiles, uint32_t tile) {
+    __shared__ uint32_t cnt[RMDA_MAX_EXPERTS];
+    __shared__ uint32_t end[RMDA_MAX_EXPERTS];  // inclusive padded ends
+    __shared__ uint32_t sbuf[1024 / RMDA_WAVE];
+    count_block<VEC>(idx, npairs, experts, count, cnt);
+    __syncthreads();
+    const uint32_t e = threadIdx.x;
+    const uint32_t p = e < experts ? (cnt[e] + tile - 1u) / tile * tile : 0u;
+    uint32_t total;
+    const uint32_t o = block_exscan<1024>(p, sbuf, &total);
+    if (e < experts) {
+        off[e] = o;
+        end[e] = o + p;
+    }
+    __syncthreads();
+    fill_tiles(end, tiles, n_tiles, experts, tile, 1024);
 }
 
 }  // namespace
@@ -845,6 +884,18 @@ hipError_t rmda_launch_count(hipStream_t s, const uint32_t *idx, uint32_t npairs
         hipLaunchKernelGGL(count_kernel<true>, dim3(1), dim3(1024), 0, s, idx, npairs, experts, count);
     } else {
         hipLaunchKernelGGL(count_kernel<false>, dim3(1), dim3(1024), 0, s, idx, npairs, experts, count);
+    }
+    return hipGetLastError();
+}
+
+hipError_t rmda_launch_count_scan(hipStream_t s, const uint32_t *idx, uint32_t npairs, uint32_t experts,
+                                  uint32_t *count, uint32_t *off, uint32_t *tiles, uint32_t n_tiles, uint32_t tile) {
+    if ((reinterpret_cast<uintptr_t>(idx) & 15u) == 0) {
+        hipLaunchKernelGGL(count_scan_kernel<true>, dim3(1), dim3(1024), 0, s, idx, npairs, experts, count, off, tiles,
+                           n_tiles, tile);
+    } else {
+        hipLaunchKernelGGL(count_scan_kernel<false>, dim3(1), dim3(1024), 0, s, idx, npairs, experts, count, off,
+                           tiles, n_tiles, tile);
     }
     return hipGetLastError();
 }
