@@ -1230,6 +1230,19 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // fp16 expert rows (2 * inter <= d).
     const bool cast_in_down = x32 && strip_dn && 2 * I <= d && rmda_gemm_strip_casts(items_max, d);
     float *const hp32 = x32 ? at<float>(ws, p.ye + (cast_in_down ? (size_t)p.groups_rows * d * 2 : 0)) : nullptr;
+    // Streaming tile: experts averaging up to 40 rows run it with one barrier
+    // per stage.  The second one keeps a fifth stage in flight, which pays
+    // while the MFMAs of a stage are long (experts of 48 rows and more) and
+    // costs more than it gives when they are short.  Layer, MI355X: 512
+    // experts top-10, hidden 2560, width 640: 10 rows 944 -> 920 us, 20 rows
+    // 1000 -> 976, 40 rows 1056 -> 1048 (from fp32 activations 1156 -> 1150),
+    // 51 rows 1237 -> 1247; hidden 2048, width 512: 20 rows 664 -> 651, 40
+    // rows 694 -> 695; 128 experts, width 768: 8 rows 213 -> 211.5, 40 rows
+    // 240 -> 241, 49 rows 247 -> 250.
+    rmda_gemm2_cfg_t g2 = ctx->g2;
+    if (g2.spec == 6 && (uint64_t)T * K <= 40ull * E) {
+        g2.spec = 4;
+    }
     rmda_gemm_args_t g{};
     g.items = at<uint32_t>(ws, p.items);
     g.n_items = at<uint32_t>(ws, p.n_items);
@@ -1256,13 +1269,12 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
         g.inter = I;
         g.out = hp;
         g.ldo = I;
-        // The default configuration streams gate_up's gathered rows through a
-        // ring of two-K-step slots when experts average 32 rows or more
-        // (configs 3 and 5: -2.1% / -2.4% gate_up); at decode sizes, where
-        // almost every activation row is padding, the single ring is faster
-        // (config 2: +5% with the activation ring).
-        rmda_gemm2_cfg_t gu = ctx->g2;
-        if (gu.spec == 6 && (uint64_t)T * K >= 32ull * E) {
+        // With more rows the default configuration streams gate_up's gathered
+        // rows through a ring of two-K-step slots (configs 3 and 5: -2.1% /
+        // -2.4% gate_up; at decode sizes, where almost every activation row
+        // is padding, the single ring is faster).
+        rmda_gemm2_cfg_t gu = g2;
+        if (gu.spec == 6) {
             gu.spec = 7;
         }
         // the compute tile first (it has work only when the rank kernel cut
@@ -1332,7 +1344,7 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
             g.fc.hc = rmda_hc_t{args->h, args->inj, args->inj_stride, args->inj_off, args->hc};
         }
         rc = strip_dn ? hip_check(ctx, rmda_launch_gemm_strip(s, &g, items_max, item_rows), "layer down")
-                      : gemm_pair(ctx, s, g, ctx->g2, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode,
+                      : gemm_pair(ctx, s, g, g2, packed != nullptr, at<uint32_t>(ws, p.n_items_hot), tile_mode,
                                   "layer down");
     }
     if (rc == RMDA_OK) {

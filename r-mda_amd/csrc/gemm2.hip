@@ -41,7 +41,7 @@
 //   * gemm2_kernel: every MFMA wave also issues its share of each stage's
 //     DMA, between its MFMA groups (HF-layout weights, and measurement
 //     variants for packed ones).
-//   * gemm4_kernel (gate_up when experts average 32 rows or more): as
+//   * gemm4_kernel (gate_up when experts average over 40 rows): as
 //     gemm3_kernel below, with the gathered activation rows in a ring of
 //     their own, two K steps per slot, so each row is one 128-byte line per
 //     pair of K steps.
@@ -59,6 +59,7 @@
 //     us; configs 2 and 4 are unchanged and the teacher's shape from fp32
 //     activations 0.4% slower.  Most of the gain shows in the next call's
 //     gate_up, not in down itself (at 512 experts down is 2% slower).
+//     Experts averaging up to 40 rows run with one barrier per stage.
 #include "common.h"
 #include "gemm_sched.h"
 
@@ -1209,9 +1210,9 @@ hipError_t launch_mode(hipStream_t s, const rmda_gemm_args_t *a, const rmda_gemm
 
 // Variant 0 is the default: the fastest configuration measured on MI355X at
 // the benchmark shapes (packed weights run the dedicated-issue kernel, with
-// the second per-stage barrier for both GEMMs, and the layer switches
-// gate_up to the activation-ring kernel when experts average 32 rows or
-// more; HF-layout weights always run gemm2_kernel).  The others are kept for
+// the second per-stage barrier for both GEMMs when experts average over 40
+// rows, where the layer also switches gate_up to the activation-ring kernel,
+// and one barrier otherwise; HF-layout weights always run gemm2_kernel).  The others are kept for
 // measurement.  LDS per workgroup =
 // STAGES * (192 + BN) * BK * 2.
 rmda_gemm2_cfg_t rmda_gemm2_variant(int variant) {
