@@ -766,7 +766,8 @@ struct mm_swiglu_t {
 };
 static int moe_mm(rmda_moe_ctx_t *ctx, const rmda_pc_moe_mm_t *pc, const uint16_t *a, const uint16_t *b, float *c,
                   const uint32_t *amax, const uint32_t *tiles, const uint32_t *live_off,
-                  const uint32_t *live_count, mm_swiglu_t *swi = nullptr) {
+                  const uint32_t *live_count, mm_swiglu_t *swi = nullptr, uint32_t live_experts = 0,
+                  uint32_t live_rows = 0) {
     if (swi != nullptr) {
         swi->fused = false;
     }
@@ -804,6 +805,8 @@ static int moe_mm(rmda_moe_ctx_t *ctx, const rmda_pc_moe_mm_t *pc, const uint16_
     if (rmda_ref_mm_supported(&g)) {
         g.live_off = live_off;
         g.live_count = live_count;
+        g.live_experts = live_experts;
+        g.live_rows = live_rows;
         if (swi != nullptr && swi->out != nullptr) {
             g.f32_swiglu = 1;
             g.so = swi->so;
@@ -1887,10 +1890,11 @@ int rmda_qwen_moe_layout(const rmda_qwen_moe_t *q, rmda_qwen_moe_layout_t *out) 
 
 namespace {
 
-// mda_qwen_moe_mm's work; live = true (the recording) leaves the padding
-// rows of each segment out of the GEMM, since nothing reads their results
+// mda_qwen_moe_mm's work; live_pairs > 0 (the recording, its routed pairs)
+// leaves the padding rows of each segment out of the GEMM, since nothing reads
+// their results
 int qwen_moe_mm(rmda_qwen_moe_t *q, const uint16_t *a, uint32_t sa, const uint16_t *w, float *out, uint32_t m,
-                uint32_t n, uint32_t k, bool live, mm_swiglu_t *swi = nullptr) {
+                uint32_t n, uint32_t k, uint32_t live_pairs, mm_swiglu_t *swi = nullptr) {
     ShimPlan p;
     int rc = shim_enter(q, "rmda_qwen_moe_mm", &p);
     if (rc != RMDA_OK) {
@@ -1901,14 +1905,16 @@ int qwen_moe_mm(rmda_qwen_moe_t *q, const uint16_t *a, uint32_t sa, const uint16
     }
     const rmda_pc_moe_mm_t pc{m, n, k, sa, RMDA_NO_SLOT};
     return moe_mm(q->ctx, &pc, a, w, out, scr<uint32_t>(q, p.amax), scr<uint32_t>(q, p.tiles),
-                  live ? scr<uint32_t>(q, p.off) : nullptr, live ? scr<uint32_t>(q, p.count) : nullptr, swi);
+                  live_pairs > 0 ? scr<uint32_t>(q, p.off) : nullptr,
+                  live_pairs > 0 ? scr<uint32_t>(q, p.count) : nullptr, swi, live_pairs > 0 ? q->experts : 0u,
+                  live_pairs);
 }
 
 }  // namespace
 
 int rmda_qwen_moe_mm(rmda_qwen_moe_t *q, const uint16_t *a, uint32_t sa, const uint16_t *w, float *out, uint32_t m,
                      uint32_t n, uint32_t k) {
-    return qwen_moe_mm(q, a, sa, w, out, m, n, k, false);
+    return qwen_moe_mm(q, a, sa, w, out, m, n, k, 0);
 }
 
 namespace {
@@ -2086,8 +2092,8 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
     }
     mm_swiglu_t swi{scr<float>(q, p.hp), sh, false};
     if (rc == RMDA_OK) {
-        rc = qwen_moe_mm(q, scr<uint16_t>(q, p.xp), sx, q->w_gate_up, scr<float>(q, p.g), mrows, 2 * I, d, true,
-                         &swi);
+        rc = qwen_moe_mm(q, scr<uint16_t>(q, p.xp), sx, q->w_gate_up, scr<float>(q, p.g), mrows, 2 * I, d,
+                         rows * K, &swi);
     }
     // over the rows that hold routed pairs only: in the reference the padding
     // rows of each 128-row segment are zero in g (xp's zero rows), so their
@@ -2107,7 +2113,7 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
                        "moe_rec hp cast");
     }
     if (rc == RMDA_OK) {
-        rc = qwen_moe_mm(q, scr<uint16_t>(q, p.hp16), sh, q->w_down, scr<float>(q, p.ye), mrows, d, I, true);
+        rc = qwen_moe_mm(q, scr<uint16_t>(q, p.hp16), sh, q->w_down, scr<float>(q, p.ye), mrows, d, I, rows * K);
     }
     // A8: the shared expert as one-expert grouped GEMMs over the padded rows
     // (src/qwen.c:879-886); rows past `rows` hold stale data and are unused

@@ -516,6 +516,11 @@ struct rmda_gemm_args_t {
     // (e = tiles[t]) are then neither computed nor stored
     const uint32_t *live_off;
     const uint32_t *live_count;
+    // F32 mode, optional with live_count: the experts it counts, where every
+    // used row lies in one of their segments, and a bound of those rows; 0
+    // where only tiles says which expert a row belongs to
+    uint32_t live_experts;
+    uint32_t live_rows;
     // F32 mode, optional: out is silu(C[:, j]) * C[:, n_w/2 + j] (qwen_elem
     // op 0 on C) as [m][n_w/2] fp32, and amax[so] takes the absmax of what is
     // stored (atomicMax of the bits, as rmda_launch_elem_absmax); needs the

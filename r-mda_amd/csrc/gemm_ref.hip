@@ -36,7 +36,8 @@
 //     count their own loads only (gate_up 327 -> 260 us), and C goes out with
 //     non-temporal stores, written once and not read again here
 //     (260 -> 247 us).
-//   * LIVE (the recording's own calls, rmda_gemm_args_t::live_count): a
+//   * LIVE (the recording's shared expert, and its routed ones where
+//     ref_live_kernel's item list is too small; live_count): a
 //     tile's rows past its segment's routed rows are padding whose results
 //     nothing reads, so a wave whose 64 rows are all padding reads no
 //     fragments and runs no MFMAs, padding rows are not stored, and their A
@@ -46,7 +47,7 @@
 //     gate_up about 7 us faster without that, 238 -> 231 and 231 -> 224 us
 //     on two boxes, its down unchanged).  At T = 2048,
 //     128 experts, top-8 a third of the used tiles' rows are padding.
-//   * SWI (rmda_gemm_args_t::f32_swiglu, the recording's gate_up): the N
+//   * SWI (rmda_gemm_args_t::f32_swiglu, the recording's gate_ups): the N
 //     tile is 128 gate columns j and their 128 up columns n_w/2 + j, laid out
 //     so that each MFMA wave holds 32 of each for the same 32 outputs (LDS
 //     rows 64w .. 64w+31 gate, 64w+32 .. 64w+63 up); the epilogue writes
@@ -350,6 +351,355 @@ __global__ __launch_bounds__(768) void ref_mm_kernel(rmda_gemm_args_t g) {
     }
 }
 
+// The recording's routed GEMMs (LIVE above) with work items of up to 192 rows
+// of one expert where that saves rounds, else of up to 128.
+//
+// A round of tasks (one per CU) takes as long as a full one, and with 128-row
+// tiles the few rows past an expert's first 128 are a task of their own (2048
+// tokens, 128 experts, top-8: half of the experts have 1 to 32 of them), so
+// every workgroup counts both kinds of items from the experts' row counts and
+// takes the height that needs less time.  Measured on MI355X: the whole
+// recording at that size 453 -> 405 us; 64 experts, 2300 tokens 388 -> 343 us;
+// 16 experts top-2, 2560 x 1024, 2048 tokens 218 -> 187 us.
+//
+//   * 12 MFMA waves = 3 (M) x 4 (N) of 64 x 64 and 4 issue waves.  Up to 192
+//     rows x 64 of A in a ring of two slots, or 128 x 64 in one of three, and
+//     256 x 64 of B in a ring of three: 144 KiB of LDS either way.
+//   * 16 waves leave 128 VGPRs: both K halves' fragments use the same
+//     registers, so the second half is read behind the first one's MFMAs.
+//   * Lines, swizzle, K start per expert, K order and epilogues are as above,
+//     so results are bitwise those of the 128-row tiles.
+constexpr uint32_t WM = 192;
+constexpr uint32_t WMW = 12;
+constexpr uint32_t WIW = 4;
+constexpr uint32_t W_MAX_ITEMS = 2048;
+constexpr uint32_t W_B_BYTES = RN * RK * 2;                                // 32 KiB
+constexpr uint32_t W_SMEM = 2 * WM * RK * 2 + 3 * W_B_BYTES;               // 144 KiB
+static_assert(2 * WM == 3 * RM, "both A rings have the same size");
+
+struct live_list_t {
+    uint16_t e[W_MAX_ITEMS];  // item: expert
+    uint16_t c[W_MAX_ITEMS];  // and H-row chunk of its rows
+};
+
+template <uint32_t H, bool SWI>
+__device__ __forceinline__ void ref_live_tasks(const rmda_gemm_args_t &g, uint8_t *smem, const live_list_t &il,
+                                               uint32_t n_items, uint32_t *swi_max, uint32_t *swi_done) {
+    constexpr uint32_t CH = RK / 8;
+    constexpr uint32_t RPI = 64 / CH;
+    constexpr uint32_t A_BYTES = H * RK * 2;
+    constexpr uint32_t B_BYTES = W_B_BYTES;
+    constexpr uint32_t A_SLOTS = H == WM ? 2 : 3;
+    constexpr uint32_t B_SLOTS = 3;
+    constexpr uint32_t LA = H / RPI / WIW;      // A instructions per issue wave and stage: 6 or 4
+    constexpr uint32_t LB = RN / RPI / WIW;     // 8 B instructions
+    static_assert(LA * RPI * WIW == H && LB * RPI * WIW == RN, "DMA split");
+    static_assert(2 * LA + 2 * LB < 64, "vmcnt range");
+    uint8_t *const aring = smem;
+    uint8_t *const bring = smem + A_SLOTS * A_BYTES;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid % RMDA_WAVE;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid / RMDA_WAVE);
+    const uint32_t ntiles = g.n_w / RN;
+    const chunk_sched_t sched(n_items, ntiles);
+    const uint32_t ntask = sched.ntask;
+    if (ntask == 0) {
+        return;
+    }
+    const uint32_t steps = g.k / RK;
+    const uint32_t nstage = ntask * steps;
+    const const_u32p off = (const_u32p)g.live_off;
+    const const_u32p count = (const_u32p)g.live_count;
+
+    if (w >= WMW) {
+        // ================= issue waves =================
+        const uint32_t dw = w - WMW;
+        const uint32_t lrow = lane / CH;
+        const uint32_t lch = lane % CH;
+        // A and B run at different distances ahead, each with its own task
+        const uint16_t *a_src[LA];
+        const uint16_t *b_src[LB];
+        uint32_t a_rot = 0, b_rot = 0;
+        auto setup_a = [&](uint32_t q) __attribute__((always_inline)) {
+            uint32_t nt;
+            const uint32_t ci = sched.item(q, nt);
+            const uint32_t e = __builtin_amdgcn_readfirstlane(il.e[ci]);
+            const uint32_t r0 = __builtin_amdgcn_readfirstlane(il.c[ci]) * H;
+            const uint32_t lv = min(count[e] - r0, H);  // > 0
+            a_rot = e * 5 % steps;
+#pragma unroll
+            for (uint32_t j = 0; j < LA; j += 1) {
+                const uint32_t r = (dw * LA + j) * RPI + lrow;
+                const uint32_t ra = r < lv ? r : 0u;  // rows past the segment re-read the first
+                a_src[j] = g.a + (size_t)(off[e] + r0 + ra) * g.lda + (lch ^ swz<RK>(r)) * 8;
+            }
+        };
+        auto setup_b = [&](uint32_t q) __attribute__((always_inline)) {
+            uint32_t nt;
+            const uint32_t ci = sched.item(q, nt);
+            const uint32_t e = __builtin_amdgcn_readfirstlane(il.e[ci]);
+            b_rot = e * 5 % steps;
+            const uint16_t *wg = g.w + (size_t)e * g.n_w * g.k;
+#pragma unroll
+            for (uint32_t j = 0; j < LB; j += 1) {
+                const uint32_t n = (dw * LB + j) * RPI + lrow;
+                const uint32_t wr = SWI ? (n % 64 < 32 ? 0u : g.n_w / 2) + nt * (RN / 2) + (n / 64) * 32 + n % 32
+                                        : nt * RN + n;
+                b_src[j] = wg + (size_t)wr * g.k + (lch ^ swz<RK>(n)) * 8;
+            }
+        };
+        uint32_t a_task = 0, a_s = 0, a_slot = 0;
+        uint32_t b_task = 0, b_s = 0, b_slot = 0;
+        setup_a(0);
+        setup_b(0);
+        auto issue_a = [&]() __attribute__((always_inline)) {
+            if (a_s == steps) {
+                a_task += 1;
+                a_s = 0;
+                setup_a(a_task);
+            }
+            uint8_t *base = aring + a_slot * A_BYTES;
+            const uint32_t kk = a_s + a_rot < steps ? a_s + a_rot : a_s + a_rot - steps;
+#pragma unroll
+            for (uint32_t j = 0; j < LA; j += 1) {
+                __builtin_amdgcn_global_load_lds((const void *)(a_src[j] + kk * RK),
+                                                 (lds_void_t *)(base + (dw * LA + j) * RPI * (RK * 2)), 16, 0, 0);
+            }
+            a_s += 1;
+            a_slot = a_slot + 1 == A_SLOTS ? 0 : a_slot + 1;
+        };
+        auto issue_b = [&]() __attribute__((always_inline)) {
+            if (b_s == steps) {
+                b_task += 1;
+                b_s = 0;
+                setup_b(b_task);
+            }
+            uint8_t *base = bring + b_slot * B_BYTES;
+            const uint32_t kk = b_s + b_rot < steps ? b_s + b_rot : b_s + b_rot - steps;
+#pragma unroll
+            for (uint32_t j = 0; j < LB; j += 1) {
+                __builtin_amdgcn_global_load_lds((const void *)(b_src[j] + kk * RK),
+                                                 (lds_void_t *)(base + (dw * LB + j) * RPI * (RK * 2)), 16, 0, 0);
+            }
+            b_s += 1;
+            b_slot = b_slot + 1 == B_SLOTS ? 0 : b_slot + 1;
+        };
+        if constexpr (A_SLOTS == B_SLOTS) {
+            for (uint32_t st = 0; st < 3 && st < nstage; st += 1) {
+                issue_a();
+                issue_b();
+            }
+            for (uint32_t gs = 0; gs < nstage; gs += 1) {
+                wait_after<LA + LB>(min(nstage - 1 - gs, 2u));
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_s_barrier();
+                if (gs + 3 < nstage) {
+                    issue_a();
+                    issue_b();
+                }
+            }
+        } else {
+            // issue order A0 B0 A1 B1 B2, then A(s+2) B(s+3) once stage s is
+            // free: behind the later of A(s) and B(s) lie A(s+1), B(s+1) and
+            // B(s+2) in some order, less at the end of the last task
+            issue_a();
+            issue_b();
+            if (nstage > 1) {
+                issue_a();
+                issue_b();
+            }
+            if (nstage > 2) {
+                issue_b();
+            }
+            for (uint32_t gs = 0; gs < nstage; gs += 1) {
+                const uint32_t later = nstage - 1 - gs;
+                if (later >= 2) {
+                    wait_vm<LA + 2 * LB>();
+                } else if (later == 1) {
+                    wait_vm<LA + LB>();
+                } else {
+                    wait_vm<0>();
+                }
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_s_barrier();
+                if (gs + 2 < nstage) {
+                    issue_a();
+                }
+                if (gs + 3 < nstage) {
+                    issue_b();
+                }
+            }
+        }
+        return;
+    }
+
+    // ================= MFMA waves =================
+    const uint32_t wm = w / 4;
+    const uint32_t wn = w % 4;
+    const uint32_t fr = lane % 16;
+    const uint32_t fq = lane / 16;
+    const uint32_t a_row = (wm * 64 + fr) * (RK * 2);
+    const uint32_t b_row = (wn * 64 + fr) * (RK * 2);
+    const uint32_t c0 = ((0u + fq) ^ swz<RK>(fr)) * 16;
+    const uint32_t c1 = ((4u + fq) ^ swz<RK>(fr)) * 16;
+    const uint32_t rq = 4 * fq;
+    const float sc = 1.0f / (ref_slot_scale(g.amax, g.sa) * ref_slot_scale(g.amax, g.sb));
+    float *C = reinterpret_cast<float *>(g.out);
+    floatx4_t acc[4][4];
+    float amx = 0.0f;
+    uint32_t kc = 0, ks = 0, abuf = 0, bbuf = 0;
+    uint32_t lrows = 0, row0 = 0, nt = 0;
+    bool live = false;
+    for (uint32_t gs = 0; gs < nstage; gs += 1) {
+        lds_barrier();
+        if (ks == 0) {
+            const uint32_t ci = sched.item(kc, nt);
+            const uint32_t e = __builtin_amdgcn_readfirstlane(il.e[ci]);
+            const uint32_t r0 = __builtin_amdgcn_readfirstlane(il.c[ci]) * H;
+            lrows = min(count[e] - r0, H);
+            row0 = off[e] + r0;
+            live = lrows > wm * 64;
+#pragma unroll
+            for (int i = 0; i < 4; i += 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j += 1) {
+                    acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        }
+        const uint8_t *ab = aring + abuf * A_BYTES + a_row;
+        const uint8_t *bb = bring + bbuf * B_BYTES + b_row;
+        abuf = abuf + 1 == A_SLOTS ? 0 : abuf + 1;
+        bbuf = bbuf + 1 == B_SLOTS ? 0 : bbuf + 1;
+        half8_t fa[4], fb[4];
+        auto read = [&](uint32_t c) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 1) {
+                fa[i] = *reinterpret_cast<const half8_t *>(ab + i * 16 * (RK * 2) + c);
+                fb[i] = *reinterpret_cast<const half8_t *>(bb + i * 16 * (RK * 2) + c);
+            }
+        };
+        auto mma = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j += 1) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+                }
+            }
+        };
+        if (live) {
+            read(c0);
+            mma();
+            read(c1);
+        }
+        lds_barrier();  // the stage is read: the issue waves may refill its buffers
+        if (live) {
+            mma();
+        }
+        if (live && ks == steps - 1) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 1) {
+#pragma unroll
+                for (int v = 0; v < 4; v += 1) {
+                    const uint32_t rt = wm * 64 + i * 16 + rq + v;
+                    if (rt >= lrows) {
+                        continue;
+                    }
+                    const size_t r = row0 + rt;
+                    if constexpr (SWI) {
+#pragma unroll
+                        for (int j = 0; j < 2; j += 1) {
+                            const float h = rmda_swiglu(acc[i][j][v] * sc, acc[i][j + 2][v] * sc);
+                            amx = fmaxf(amx, fabsf(h));
+                            __builtin_nontemporal_store(h, &C[r * g.ldo + nt * (RN / 2) + wn * 32 + j * 16 + fr]);
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; j += 1) {
+                            __builtin_nontemporal_store(acc[i][j][v] * sc,
+                                                        &C[r * g.ldo + nt * RN + wn * 64 + j * 16 + fr]);
+                        }
+                    }
+                }
+            }
+        }
+        ks += 1;
+        if (ks == steps) {
+            ks = 0;
+            kc += 1;
+        }
+    }
+    if constexpr (SWI) {
+        const uint32_t m = rmda_wave_red_u32<true>(__builtin_bit_cast(uint32_t, amx));
+        if (lane == 0) {
+            atomicMax(swi_max, m);
+            if (atomicAdd(swi_done, 1u) == WMW - 1 && g.so != RMDA_NO_SLOT) {
+                atomicMax(const_cast<uint32_t *>(&g.amax[g.so]), atomicMax(swi_max, 0u));
+            }
+        }
+    }
+}
+
+template <bool SWI>
+__global__ __launch_bounds__((WMW + WIW) * RMDA_WAVE) void ref_live_kernel(rmda_gemm_args_t g) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[W_SMEM];
+    __shared__ live_list_t il;
+    __shared__ uint32_t wsum[WMW + WIW];
+    __shared__ uint32_t swi_max, swi_done;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid % RMDA_WAVE;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid / RMDA_WAVE);
+    if (SWI && tid == 0) {
+        swi_max = 0u;
+        swi_done = 0u;
+    }
+    // thread e < experts counts and places expert e's items, in expert order:
+    // both counts scanned in one word (each at most W_MAX_ITEMS)
+    const uint32_t cnt = tid < g.live_experts ? g.live_count[tid] : 0u;
+    const uint32_t ni = (cnt + RM - 1u) / RM | (cnt + WM - 1u) / WM << 16;
+    uint32_t pre = ni;
+#pragma unroll
+    for (uint32_t o = 1; o < RMDA_WAVE; o <<= 1) {
+        const uint32_t v = __shfl_up(pre, o);
+        pre += lane >= o ? v : 0u;
+    }
+    if (lane == RMDA_WAVE - 1) {
+        wsum[w] = pre;
+    }
+    __syncthreads();
+    uint32_t total = 0;
+    uint32_t at = pre - ni;
+    for (uint32_t q = 0; q < WMW + WIW; q += 1) {
+        at += q < w ? wsum[q] : 0u;
+        total += wsum[q];
+    }
+    total = __builtin_amdgcn_readfirstlane(total);
+    const uint32_t ntiles = g.n_w / RN;
+    const uint32_t r_lo = ((total & 0xffffu) * ntiles + gridDim.x - 1u) / gridDim.x;
+    const uint32_t r_hi = ((total >> 16) * ntiles + gridDim.x - 1u) / gridDim.x;
+    // Rounds of either kind.  A 192-row task costs up to 1.25 (gate_up) or 1.2
+    // (down) of a 128-row one where the weights' bytes dominate, up to 1.5
+    // where the MFMAs do.  Measured on MI355X, 2048 x 768, top-8, 64 experts,
+    // 128 rows against 192: gate_up at 5 rounds against 3 (2300 tokens) -22 to
+    // -33 us of 389, 4 against 3 (1900) -11 of 352, 3 against 2 (1100) -8 of
+    // 267 and (1400) +2 of 274, 5 against 4 (3000) +14 of 464, 6 against 5
+    // (3500) +9; down at 5 against 4 (2048) -8, 6 against 4 (2600) -5, 4
+    // against 3 (1400) +8 and (1536) 0, equal rounds +5 to +7.
+    const bool tall = SWI ? 5u * r_hi < 4u * r_lo : 6u * r_hi < 5u * r_lo;
+    const uint32_t sh = tall ? 16u : 0u;
+    for (uint32_t c = 0; c < (ni >> sh & 0xffffu); c += 1) {
+        il.e[(at >> sh & 0xffffu) + c] = (uint16_t)tid;
+        il.c[(at >> sh & 0xffffu) + c] = (uint16_t)c;
+    }
+    __syncthreads();
+    if (tall) {
+        ref_live_tasks<WM, SWI>(g, smem, il, total >> 16, &swi_max, &swi_done);
+    } else {
+        ref_live_tasks<RM, SWI>(g, smem, il, total & 0xffffu, &swi_max, &swi_done);
+    }
+}
+
 }  // namespace
 
 bool rmda_ref_mm_supported(const rmda_gemm_args_t *a) {
@@ -368,6 +718,15 @@ hipError_t rmda_launch_ref_mm(hipStream_t s, const rmda_gemm_args_t *a, uint32_t
     if ((a->live_count != nullptr) != (a->live_off != nullptr) ||
         (a->f32_swiglu && (a->amax == nullptr && a->so != RMDA_NO_SLOT))) {
         return hipErrorInvalidValue;
+    }
+    if (a->live_count != nullptr && a->live_experts > 0 && a->live_experts <= (WMW + WIW) * RMDA_WAVE &&
+        a->live_rows / RM + a->live_experts <= W_MAX_ITEMS) {
+        if (a->f32_swiglu) {
+            hipLaunchKernelGGL(ref_live_kernel<true>, gr, dim3((WMW + WIW) * RMDA_WAVE), 0, s, *a);
+        } else {
+            hipLaunchKernelGGL(ref_live_kernel<false>, gr, dim3((WMW + WIW) * RMDA_WAVE), 0, s, *a);
+        }
+        return hipGetLastError();
     }
     if (a->f32_swiglu) {
         if (a->live_count != nullptr) {

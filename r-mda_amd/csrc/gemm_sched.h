@@ -122,18 +122,28 @@ struct task_sched_t {
 // Contiguous schedule: round q's tasks [q*G, (q+1)*G) in list order (item
 // major, N tile minor) are cut into eight runs of G/8, one per XCD, so the
 // CUs of an XCD work on adjacent items, i.e. on the same expert's weight
-// tiles and neighbouring row blocks, and share both through their L2.
+// tiles and neighbouring row blocks, and share both through their L2.  A last
+// round of fewer than G tasks is cut into eight shorter runs, so that all
+// XCDs read its weights (dealt by whole runs it would sit on the first ones:
+// the recording with 8 experts top-2, 2560 x 1024, 512 tokens 110 -> 103 us,
+// 64 experts top-8, 2048 x 768, 2048 tokens, 128-row tiles 370 -> 357 us).
 struct chunk_sched_t {
-    uint32_t G, pos, ntiles, ntask;
+    uint32_t G, pos, last, full, ntiles, ntask;
     __device__ __forceinline__ chunk_sched_t(uint32_t n_items, uint32_t nt) {
         G = gridDim.x;
-        pos = (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u;
+        const uint32_t x = blockIdx.x % 8u;
+        const uint32_t j = blockIdx.x / 8u;
+        pos = x * (G / 8u) + j;
         ntiles = nt;
         const uint32_t total = n_items * nt;
-        ntask = total / G + (pos < total % G ? 1u : 0u);
+        const uint32_t rem = total % G;
+        const uint32_t per = (rem + 7u) / 8u;
+        full = total / G;
+        last = x * per + j;
+        ntask = full + (j < per && last < rem ? 1u : 0u);
     }
     __device__ __forceinline__ uint32_t item(uint32_t q, uint32_t &nt) const {
-        const uint32_t t = q * G + pos;
+        const uint32_t t = q * G + (q < full ? pos : last);
         const uint32_t k = t / ntiles;
         nt = t - k * ntiles;
         return k;
