@@ -36,6 +36,7 @@ CASES = [
     case(64, 1280, 300, 3, 512, skew=True),       # most experts without rows
     case(1, 768, 174, 1, 256),                    # fp32 activations: down casts the SwiGLU output
     case(3, 512, 182, 4, 256, shared=True), case(70, 512, 3, 1, 256), case(40, 512, 2, 2, 256, shared=True),
+    case(1536, 512, 8, 2, 1024), case(975, 512, 13, 10, 384),  # large experts: strips in down only; in neither GEMM
 ]
 
 
