@@ -516,11 +516,6 @@ struct rmda_gemm_args_t {
     // (e = tiles[t]) are then neither computed nor stored
     const uint32_t *live_off;
     const uint32_t *live_count;
-    // F32 mode, optional with live_count: the experts it counts, where every
-    // used row lies in one of their segments, and a bound of those rows; 0
-    // where only tiles says which expert a row belongs to
-    uint32_t live_experts;
-    uint32_t live_rows;
     // F32 mode, optional: out is silu(C[:, j]) * C[:, n_w/2 + j] (qwen_elem
     // op 0 on C) as [m][n_w/2] fp32, and amax[so] takes the absmax of what is
     // stored (atomicMax of the bits, as rmda_launch_elem_absmax); needs the
@@ -544,15 +539,23 @@ struct rmda_gemm_args_t {
     const uint32_t *yscale;
     float *ye32;
     const uint32_t *ye_bound;
+    // F16, fp16 rows, packed weights: non-zero asks for non-temporal row
+    // stores (both tiles' default configurations)
+    uint32_t ye_nt;
+    // What two kernels read lies last: in the middle it moved the others'
+    // argument offsets and with them their scalar loads' grouping (compute
+    // tile, 21 touched experts of 128, 2048 tokens: layer 239.1 -> 240.0 us).
+    // F32 mode, optional with live_count: the experts it counts, where every
+    // used row lies in one of their segments, and a bound of those rows; 0
+    // where only tiles says which expert a row belongs to
+    uint32_t live_experts;
+    uint32_t live_rows;
     // Strip kernel, F16: with a32 set, A is the fp32 SwiGLU output (same
     // blocked index) and is cast on the way with the slot of the partial
     // absmax words a_parts, whose fold goes to *a_slot.
     const float *a32;
     const uint32_t *a_parts;
     uint32_t *a_slot;
-    // F16, fp16 rows, packed weights: non-zero asks for non-temporal row
-    // stores (both tiles' default configurations)
-    uint32_t ye_nt;
 };
 hipError_t rmda_launch_gemm(hipStream_t s, const rmda_gemm_args_t *a);
 // gemm_ref.hip: the F32 (reference matmul_f16_moe) contract on the
