@@ -613,8 +613,10 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
 // lda, and for F16 the sorted rows * lda, below 2^32 elements.
 // rmda_gemm_strip_pays: the rule for npairs routed rows over `groups` experts
 // (shared one included).
+// rmda_gemm_strip_waves: waves (= workgroups) of a launch.
 // rmda_gemm_strip_casts: whether down should cast the fp32 SwiGLU output
 // itself (a32).
+uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w);
 bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w);
 bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k);
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows);

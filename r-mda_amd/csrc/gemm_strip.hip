@@ -30,6 +30,8 @@
 // Per output element the MFMA sequence and the epilogue are those of the
 // other tiles (K steps of 32 in order from a zero accumulator), so the output
 // is bitwise the same.
+#include <algorithm>
+
 #include "common.h"
 #include "gemm_sched.h"
 
@@ -72,13 +74,20 @@ struct a_frag_t<true> {
 };
 
 // One chunk of MT live 16-row groups times one strip.
-template <int MODE, int MT, int DEPTH, bool SC, bool CAST>
+template <int MODE, int MT, int DEPTH, bool SC, bool CAST, bool MANY>
 __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t row0, uint32_t rows, bool is_shared,
-                                            const uint16_t *b0, const uint16_t *b1, uint32_t col0, float scale) {
-    const uint32_t lane = threadIdx.x;
+                                            const uint16_t *wb, uint32_t col0, float scale) {
+    uint32_t lane = threadIdx.x;
+    uint32_t steps = g.k / BK;
+    if constexpr (MANY) {
+        // opaque, so that the loop over tasks keeps nothing derived from them
+        // in registers next to the ring (which would spill)
+        asm volatile("" : "+v"(lane), "+s"(steps));
+    }
     const uint32_t fr = lane % 16;
     const uint32_t fq = lane / 16;
-    const uint32_t steps = g.k / BK;
+    const uint16_t *const b0 = wb + fr * BK + (fq ^ swz<BK>(fr)) * 8;
+    const uint16_t *const b1 = b0 + (MODE == RMDA_GEMM_SWIGLU ? 32u : 16u) * BK;
     constexpr uint32_t A_STEP = MODE == RMDA_GEMM_F16 ? RMDA_HP_ROWS * BK : BK;
     uint32_t a[MT];  // element offsets from g.a (the launch checks that they fit)
 #pragma unroll
@@ -180,7 +189,32 @@ __device__ __forceinline__ void strip_chunk(const rmda_gemm_args_t &g, uint32_t 
 // the shallow ring covers at once only pays for its longer start (one token:
 // 36.1 -> 37.3 us), and a K loop shorter than the ring reads its last step
 // again (K = 256: down 15.7 -> 21.0 us).
-template <int MODE, bool DEEP, bool SC, bool CAST>
+template <int MODE, bool DEEP, bool SC, bool CAST, bool MANY>
+__device__ __forceinline__ void strip_rows(const rmda_gemm_args_t &g, uint32_t row0, uint32_t rows, bool is_shared,
+                                           const uint16_t *wb, uint32_t col0, float scale) {
+    switch ((rows + 15u) / 16u) {
+    case 1: strip_chunk<MODE, 1, DEEP ? 16 : 8, SC, CAST, MANY>(g, row0, rows, is_shared, wb, col0, scale); break;
+    case 2: strip_chunk<MODE, 2, DEEP ? 12 : 8, SC, CAST, MANY>(g, row0, rows, is_shared, wb, col0, scale); break;
+    case 3: strip_chunk<MODE, 3, DEEP ? 8 : 6, SC, CAST, MANY>(g, row0, rows, is_shared, wb, col0, scale); break;
+    default: strip_chunk<MODE, 4, DEEP ? 7 : CAST ? 5 : 6, SC, CAST, MANY>(g, row0, rows, is_shared, wb, col0, scale); break;
+    }
+}
+
+// MANY: a launch of several chunks per item whose bound on the tasks is above
+// MANY_WAVES runs that many waves, each walking its share of the tasks that
+// the work list holds.  The bound counts an item per expert and every chunk an
+// item can have; under skewed routing, where few experts hold all rows, nine
+// tasks in ten were empty, lay between the others and cost the dispatcher
+// about 0.2 ns each (512 experts top-10, hidden 2560, width 640, 199 tokens
+// with a Zipf-like bias: layer 176 -> 159 us; top-1, width 512, hidden 2048,
+// 512 tokens 72 -> 57 us).  The chunks of an item are then one wave's, one
+// after the other, unless the list has fewer than SPLIT_WAVES strips.  With one
+// chunk per item the empty tasks are the last ones and cost nothing (51 tokens
+// of the first shape 90 us either way, evenly routed 506 -> 515 us walking).
+constexpr uint32_t MANY_WAVES = 16384;
+constexpr uint32_t SPLIT_WAVES = 8192;
+
+template <int MODE, bool DEEP, bool SC, bool CAST, bool MANY>
 __global__ __launch_bounds__(RMDA_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) void strip_kernel(
     rmda_gemm_args_t g, uint32_t chunks) {
     const const_u32p items = (const_u32p)g.items;
@@ -193,65 +227,81 @@ __global__ __launch_bounds__(RMDA_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2)
             *g.a_slot = m;  // for the combine
         }
     }
-    // blockIdx.x = (slab / 8, chunk, strip, slab % 8), slabs counted over the
-    // whole work list: the strips and row chunks of a slab share an XCD's L2
+    // task = (slab / 8, chunk, strip, slab % 8), slabs counted over the whole
+    // work list: the strips and row chunks of a slab share an XCD's L2
     const uint32_t nslab = g.n_w / SLAB;
-    const uint32_t j = blockIdx.x / 8u;
-    const uint32_t jj = j / STRIPS;
-    const uint32_t gs = jj / chunks * 8u + blockIdx.x % 8u;
-    const uint32_t r0 = jj % chunks * CHUNK;
-    const uint32_t item = gs / nslab;
-    const uint32_t slab = gs - item * nslab;
-    const uint32_t strip = j % STRIPS;
-    if (item >= *(const_u32p)g.n_items) {
-        return;
+    uint32_t per = chunks;
+    if constexpr (MANY) {
+        per = *(const_u32p)g.n_items * nslab * STRIPS >= SPLIT_WAVES ? 1u : chunks;
     }
-    const uint32_t grp = items[item * 4 + 0];
-    const uint32_t row0 = items[item * 4 + 1] + r0;
-    const uint32_t n = items[item * 4 + 2];
-    if (r0 >= n) {
-        return;
-    }
-    const uint32_t rows = min(n - r0, CHUNK);
-    const uint32_t fr = threadIdx.x % 16;
-    const uint32_t fq = threadIdx.x / 16;
-    const bool is_shared = grp == g.shared_group;
-    const uint16_t *const wg = is_shared ? g.w_shared : g.w + (size_t)grp * g.n_w * g.k;
-    // weight rows of the strip: two 16-row operands.  SWIGLU: 16 gate rows
-    // and the matching up rows, 32 slab rows further; F16: 32 adjacent rows
-    const uint32_t nb = MODE == RMDA_GEMM_SWIGLU ? strip / 2u * 64u + strip % 2u * 16u : strip * 32u;
-    const uint32_t col0 = MODE == RMDA_GEMM_SWIGLU ? slab * (SLAB / 2) + strip * 16u : slab * SLAB + strip * 32u;
-    const uint16_t *const b0 =
-        wg + (size_t)slab * (g.k / BK) * STEP + nb * BK + fr * BK + (fq ^ swz<BK>(fr)) * 8;
-    const uint16_t *const b1 = b0 + (MODE == RMDA_GEMM_SWIGLU ? 32u : 16u) * BK;
-    switch ((rows + 15u) / 16u) {
-    case 1: strip_chunk<MODE, 1, DEEP ? 16 : 8, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
-    case 2: strip_chunk<MODE, 2, DEEP ? 12 : 8, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
-    case 3: strip_chunk<MODE, 3, DEEP ? 8 : 6, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
-    default: strip_chunk<MODE, 4, DEEP ? 7 : CAST ? 5 : 6, SC, CAST>(g, row0, rows, is_shared, b0, b1, col0, scale); break;
+    for (uint32_t b = blockIdx.x;; b += gridDim.x) {
+        const uint32_t j = b / 8u;
+        const uint32_t jj = j / STRIPS;
+        const uint32_t gs = jj / per * 8u + blockIdx.x % 8u;
+        const uint32_t item = gs / nslab;
+        const uint32_t slab = gs - item * nslab;
+        const uint32_t strip = j % STRIPS;
+        if (item >= *(const_u32p)g.n_items) {
+            return;
+        }
+        const uint32_t grp = items[item * 4 + 0];
+        const uint32_t item0 = items[item * 4 + 1];
+        const uint32_t n = items[item * 4 + 2];
+        const bool is_shared = grp == g.shared_group;
+        const uint16_t *const wg = is_shared ? g.w_shared : g.w + (size_t)grp * g.n_w * g.k;
+        // weight rows of the strip: two 16-row operands.  SWIGLU: 16 gate rows
+        // and the matching up rows, 32 slab rows further; F16: 32 adjacent rows
+        const uint32_t nb = MODE == RMDA_GEMM_SWIGLU ? strip / 2u * 64u + strip % 2u * 16u : strip * 32u;
+        const uint32_t col0 = MODE == RMDA_GEMM_SWIGLU ? slab * (SLAB / 2) + strip * 16u : slab * SLAB + strip * 32u;
+        const uint16_t *const wb = wg + (size_t)slab * (g.k / BK) * STEP + nb * BK;
+        for (uint32_t r0 = jj % per * CHUNK; r0 < n; r0 += per * CHUNK) {
+            strip_rows<MODE, DEEP, SC, CAST, MANY>(g, item0 + r0, min(n - r0, CHUNK), is_shared, wb, col0, scale);
+            if constexpr (!MANY) {
+                return;  // an item has at most `chunks` chunks
+            }
+        }
+        if constexpr (!MANY) {
+            return;
+        }
     }
 }
 
-template <int MODE, bool DEEP>
+uint32_t strip_tasks(uint32_t items, uint32_t item_rows, uint32_t n_w) {
+    return (items * (n_w / SLAB) + 7) / 8 * 8 * STRIPS * ((item_rows + CHUNK - 1) / CHUNK);
+}
+
+template <int MODE, bool DEEP, bool SC>
 hipError_t launch_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
     const uint32_t chunks = (item_rows + CHUNK - 1) / CHUNK;
-    const dim3 grid((items * (a->n_w / SLAB) + 7) / 8 * 8 * STRIPS * chunks);
-    const bool sc = a->hp32 != nullptr || a->ye_bound != nullptr;
-    if constexpr (MODE == RMDA_GEMM_F16 && !DEEP) {
+    const uint32_t tasks = strip_tasks(items, item_rows, a->n_w);
+    const uint32_t waves = rmda_gemm_strip_waves(items, item_rows, a->n_w);
+    if constexpr (MODE == RMDA_GEMM_F16 && !DEEP && SC) {
         if (a->a32 != nullptr) {
-            hipLaunchKernelGGL((strip_kernel<MODE, false, true, true>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+            hipLaunchKernelGGL((strip_kernel<MODE, false, true, true, false>), dim3(tasks), dim3(RMDA_WAVE), 0, s, *a,
+                               chunks);
             return hipGetLastError();
         }
     }
-    if (sc) {
-        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, true, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+    if (tasks > waves) {
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, SC, false, true>), dim3(waves), dim3(RMDA_WAVE), 0, s, *a, chunks);
     } else {
-        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, false, false>), grid, dim3(RMDA_WAVE), 0, s, *a, chunks);
+        hipLaunchKernelGGL((strip_kernel<MODE, DEEP, SC, false, false>), dim3(tasks), dim3(RMDA_WAVE), 0, s, *a, chunks);
     }
     return hipGetLastError();
 }
 
+template <int MODE, bool DEEP>
+hipError_t launch_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
+    return a->hp32 != nullptr || a->ye_bound != nullptr ? launch_strip<MODE, DEEP, true>(s, a, items, item_rows)
+                                                        : launch_strip<MODE, DEEP, false>(s, a, items, item_rows);
+}
+
 }  // namespace
+
+uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w) {
+    const uint32_t tasks = strip_tasks(items, item_rows, n_w);
+    return item_rows <= CHUNK ? tasks : std::min(tasks, MANY_WAVES);
+}
 
 bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k) {
     const uint64_t tasks = (uint64_t)items * (n_w / SLAB);  // the streaming tile's

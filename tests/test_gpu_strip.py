@@ -5,7 +5,9 @@ element, so the results are bitwise equal; the routing and output are also
 held to the oracle's tolerance.  Shapes sit at the kernel's edges: one row, the
 16-row groups and 64-row chunks (15..17, 63..65 rows on one expert), items of
 192 rows, K loops shorter than, equal to and not a multiple of the ring, slabs
-not a multiple of the 8 XCDs, and a shared expert's rows in several chunks.
+not a multiple of the 8 XCDs, a shared expert's rows in several chunks, and
+launches of fewer waves than their bound on the tasks, each walking several,
+with the chunks of an item in one wave and in several.
 """
 import pytest
 import torch
@@ -36,6 +38,8 @@ CASES = [
     case(64, 1280, 300, 3, 512, skew=True),       # most experts without rows
     case(1, 768, 174, 1, 256),                    # fp32 activations: down casts the SwiGLU output
     case(3, 512, 182, 4, 256, shared=True), case(70, 512, 3, 1, 256), case(40, 512, 2, 2, 256, shared=True),
+    # more tasks than waves: gate_up with an item's chunks in one wave, down split; few experts with rows
+    case(180, 512, 512, 10, 384, shared=True), case(180, 768, 512, 10, 384, skew=True),
     case(1536, 512, 8, 2, 1024), case(975, 512, 13, 10, 384),  # large experts: strips in down only; in neither GEMM
 ]
 
