@@ -1135,22 +1135,11 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // strip of weight rows over the streaming tile's list (gemm_strip.hip).
     // An explicit tile policy keeps its tile.
     const uint32_t item_rows = std::min(T, RMDA_GEMM2_BM);
-    const uint32_t items_max = std::min(p.npairs, E) + p.npairs / RMDA_GEMM2_BM +
-                               (p.sh_rows + RMDA_GEMM2_BM - 1) / RMDA_GEMM2_BM;
-    const uint32_t groups = E + (p.sh_rows > 0 ? 1u : 0u);
+    const uint32_t items_max = rmda_gemm_strip_items(p.npairs, E, p.sh_rows);
     const bool strip_ok = packed != nullptr && ctx->fused_combine == 0 && ctx->tile_policy == RMDA_TILE_ADAPTIVE &&
                           ctx->g2.spec == 6 && ((uint64_t)T * d | (uint64_t)p.groups_rows * I) < (1ull << 32);
-    bool strip_gu = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, 2 * I, d);
-    bool strip_dn = strip_ok && rmda_gemm_strip_pays(p.npairs + p.sh_rows, groups, items_max, d, I);
-    // One GEMM in strips keeps the other off the compute tile, which large
-    // experts want: from 192 rows on average, only where the strips replace at
-    // most a quarter round of tasks (down of 13 experts of hidden 512, width
-    // 384, 176 tasks at 746 rows each: layer 60 us without, 65 with; of 8 of
-    // width 1024, 64 tasks at 384 rows: 63 and 55 us).
-    if (strip_gu != strip_dn && p.npairs >= 192 * E &&
-        (uint64_t)items_max * ((strip_gu ? 2 * I : d) / 256) > 64) {
-        strip_gu = strip_dn = false;
-    }
+    const uint32_t strips = strip_ok ? rmda_gemm_strip_choice(T, K, E, p.sh_rows, I, d) : 0u;
+    const bool strip_gu = (strips & 1u) != 0, strip_dn = (strips & 2u) != 0;
     // Tile of the two GEMMs (0: both launch, the rank kernel decides; 1: the
     // streaming tile only; 2: the compute tile only).  No expert can be hot
     // with fewer rows than hot_min (a token adds at most one row per expert).

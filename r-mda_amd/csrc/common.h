@@ -611,14 +611,18 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
 // experts (packed weights, gemm2's bits).  items bounds *n_items, item_rows
 // (<= RMDA_GEMM2_BM) the rows of an item.  32-bit offsets into A: a_rows *
 // lda, and for F16 the sorted rows * lda, below 2^32 elements.
-// rmda_gemm_strip_pays: the rule for npairs routed rows over `groups` experts
-// (shared one included).
+// rmda_gemm_strip_choice: which of a layer's GEMMs should take it, bit 0
+// gate_up and bit 1 down, by the shape alone (sh_rows: rows of the shared
+// expert, 0 without one).
+// rmda_gemm_strip_items: the bound on its work items.
 // rmda_gemm_strip_waves: waves (= workgroups) of a launch.
 // rmda_gemm_strip_casts: whether down should cast the fp32 SwiGLU output
 // itself (a32).
 uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w);
 bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w);
-bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k);
+uint32_t rmda_gemm_strip_items(uint32_t npairs, uint32_t experts, uint32_t sh_rows);
+uint32_t rmda_gemm_strip_choice(uint32_t rows, uint32_t topk, uint32_t experts, uint32_t sh_rows, uint32_t inter,
+                                uint32_t d);
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows);
 // Packed slab height: weight rows of one N tile (256 of gate_up's 2 * inter,
 // or of down's d).

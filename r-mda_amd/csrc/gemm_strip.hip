@@ -296,14 +296,27 @@ hipError_t launch_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items
                                                         : launch_strip<MODE, DEEP, false>(s, a, items, item_rows);
 }
 
-}  // namespace
-
-uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w) {
-    const uint32_t tasks = strip_tasks(items, item_rows, n_w);
-    return item_rows <= CHUNK ? tasks : std::min(tasks, MANY_WAVES);
+// Whether strips hold up in both GEMMs where the rows may gather on few experts.
+bool strip_spread(uint32_t rows, uint32_t topk, uint32_t inter, uint32_t d) {
+    // The shape does not say how many rows the chosen experts get.  The bound
+    // takes the worst load, all tokens on the same experts: the gate_up
+    // weights that rows * topk / 64 full chunks and topk started ones read.
+    // Layer in strips against the streaming tile under a Zipf-like bias and
+    // under even routing, by these bytes.  Above 64 rows, where an expert's
+    // chunks read its weights again: 71 MB (300 experts top-3, hidden 1280,
+    // width 640, 400 tokens) 0.89 and 0.99; 101 MB (256 top-8, 2048, 768, 65)
+    // 1.21 and 0.97; 104 MB (400 top-8, 2048, 384, 200) 0.97 and 1.00; 106 MB
+    // (160 top-5, 2560, 1024, 65) 1.12 and 0.93; 126 MB (96 tokens of the
+    // second) 1.18 and 1.04; 170 MB (512 top-10, 2560, 640, 102) 1.17 and 1.03.
+    // Up to 64 rows, one chunk each: 118 MB (51 tokens of the last) 0.91 and
+    // 0.97; 201 MB (256 top-16, 2048, 768, 64) 1.16 and 1.00; 210 MB (160
+    // top-10, 2560, 1024, 64) 1.10 and 0.98.
+    return 4ull * inter * d * topk * (rows + CHUNK) / CHUNK < (rows <= CHUNK ? 192ull << 20 : 96ull << 20);
 }
 
-bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k) {
+// Whether strips beat the streaming tile in a GEMM of n_w weight rows of k for
+// npairs rows over `groups` experts (shared one included).
+bool strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, uint32_t k, bool spread) {
     const uint64_t tasks = (uint64_t)items * (n_w / SLAB);  // the streaming tile's
     // Experts average few rows: every strip is read once and the weights
     // decide.  Up to 4 rows where the streaming tile's tasks fill two rounds
@@ -311,7 +324,7 @@ bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint
     // 204 us; 8 rows, 215 -> 213 us but 85 -> 91 us under skewed routing; 16
     // rows, 225 -> 244 us), and the more the emptier its rounds are (128
     // tasks: 16 rows, 82 -> 69 us; 32 rows, 94 -> 118 us).
-    if ((uint64_t)npairs * (tasks < 512 ? tasks : 512) <= 4ull * 512 * groups) {
+    if (spread && (uint64_t)npairs * (tasks < 512 ? tasks : 512) <= 4ull * 512 * groups) {
         return true;
     }
     // Few weights for the streaming tile's workgroups: one round or less of
@@ -321,6 +334,36 @@ bool rmda_gemm_strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint
     // skewed rows: layer 63 -> 65 us).
     const uint64_t bytes = 2ull * groups * n_w * k;
     return tasks <= 256 && bytes * ((uint64_t)npairs + 32ull * groups) / (64ull * groups) <= (64ull << 20);
+}
+
+}  // namespace
+
+uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w) {
+    const uint32_t tasks = strip_tasks(items, item_rows, n_w);
+    return item_rows <= CHUNK ? tasks : std::min(tasks, MANY_WAVES);
+}
+
+uint32_t rmda_gemm_strip_items(uint32_t npairs, uint32_t experts, uint32_t sh_rows) {
+    return std::min(npairs, experts) + npairs / RMDA_GEMM2_BM + (sh_rows + RMDA_GEMM2_BM - 1) / RMDA_GEMM2_BM;
+}
+
+uint32_t rmda_gemm_strip_choice(uint32_t rows, uint32_t topk, uint32_t experts, uint32_t sh_rows, uint32_t inter,
+                                uint32_t d) {
+    const uint32_t npairs = rows * topk;
+    const uint32_t items = rmda_gemm_strip_items(npairs, experts, sh_rows);
+    const uint32_t groups = experts + (sh_rows > 0 ? 1u : 0u);
+    const bool spread = strip_spread(rows, topk, inter, d);
+    const bool gu = strip_pays(npairs + sh_rows, groups, items, 2 * inter, d, spread);
+    const bool dn = strip_pays(npairs + sh_rows, groups, items, d, inter, spread);
+    // One GEMM in strips keeps the other off the compute tile, which large
+    // experts want: from 192 rows on average, only where the strips replace at
+    // most a quarter round of tasks (down of 13 experts of hidden 512, width
+    // 384, 176 tasks at 746 rows each: layer 60 us without, 65 with; of 8 of
+    // width 1024, 64 tasks at 384 rows: 63 and 55 us).
+    if (gu != dn && npairs >= 192 * experts && (uint64_t)items * ((gu ? 2 * inter : d) / SLAB) > 64) {
+        return 0;
+    }
+    return (gu ? 1u : 0u) | (dn ? 2u : 0u);
 }
 
 bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w) {

@@ -27,3 +27,26 @@ def internal(name, restype=ctypes.c_uint32):
 ])
 def test_strip_launch_is_bounded(items, item_rows, n_w, waves):
     assert internal("rmda_gemm_strip_waves")(items, item_rows, n_w) == waves
+
+
+GATE_UP, DOWN = 1, 2
+
+
+def strips(rows, d, experts, topk, inter, shared=0):
+    """Which GEMMs of the fused layer (packed weights, default policy) take the strip kernel."""
+    return internal("rmda_gemm_strip_choice")(rows, topk, experts, rows if shared else 0, inter, d)
+
+
+@pytest.mark.parametrize("shape,want", [
+    # few rows per expert: strips, also under skewed routing
+    ((1, 2048, 128, 8, 768), 3), ((16, 2560, 512, 10, 640, 640), 3), ((51, 2560, 512, 10, 640), 3),
+    ((400, 1280, 300, 3, 640), 3), ((200, 1792, 480, 6, 512), 3), ((512, 2048, 512, 1, 512), 3),
+    # as few on average, but all on the same experts they cost more there than they gain: 9 to 24% of the layer
+    ((102, 2560, 512, 10, 640), 0), ((199, 2560, 512, 10, 640), 0), ((65, 2048, 256, 8, 768), 0),
+    ((96, 2560, 160, 5, 1024), 0), ((64, 2048, 256, 16, 768), 0), ((64, 2048, 256, 8, 768), 3),
+    # few experts: the rows on average decide, whatever their number
+    ((256, 512, 8, 2, 1024), 3), ((1536, 512, 8, 2, 1024), DOWN), ((975, 512, 13, 10, 384), 0),
+    ((2048, 2048, 128, 8, 768), 0), ((777, 2048, 128, 8, 768), 0),
+])
+def test_strip_choice(shape, want):
+    assert strips(*shape) == want
