@@ -328,12 +328,15 @@ bool strip_pays(uint32_t npairs, uint32_t groups, uint32_t items, uint32_t n_w, 
         return true;
     }
     // Few weights for the streaming tile's workgroups: one round or less of
-    // tasks, and with the 64-row chunks counted at most 64 MB moved from L2 (8 experts, hidden 512, width 1024: 64
-    // rows per expert 51 -> 34 us, 128 rows 60 -> 42 us, 256 rows' gate_up,
-    // 75 MB, 18.9 -> 27.9 us; 288 tasks of hidden 768, width 256 at 80
-    // skewed rows: layer 63 -> 65 us).
-    const uint64_t bytes = 2ull * groups * n_w * k;
-    return tasks <= 256 && bytes * ((uint64_t)npairs + 32ull * groups) / (64ull * groups) <= (64ull << 20);
+    // tasks, and with the 64-row chunks counted at most 64 MB moved from L2 (8
+    // experts, hidden 512, width 1024: 64 rows per expert 51 -> 34 us, 128
+    // rows 60 -> 42 us, 256 rows' gate_up, 75 MB, 18.9 -> 27.9 us), less where
+    // the tasks nearly fill the round.  gate_up alone in strips, layer against
+    // the streaming tile by tasks x MB: 45 x 62 0.78, 72 x 66 0.92, 116 x 50
+    // 0.98, 128 x 59 1.02, 114 x 66 1.09, 148 x 50 1.06 (0.82 under a Zipf-like
+    // bias), 138 x 67 1.09, 160 x 63 1.12 (0.89).
+    const uint64_t moved = 2ull * groups * n_w * k * ((uint64_t)npairs + 32ull * groups) / (64ull * groups);
+    return tasks <= 256 && moved <= (64ull << 20) && tasks * moved <= (8192ull << 20);
 }
 
 }  // namespace

@@ -44,7 +44,9 @@ def strips(rows, d, experts, topk, inter, shared=0):
     # as few on average, but all on the same experts they cost more there than they gain: 9 to 24% of the layer
     ((102, 2560, 512, 10, 640), 0), ((199, 2560, 512, 10, 640), 0), ((65, 2048, 256, 8, 768), 0),
     ((96, 2560, 160, 5, 1024), 0), ((64, 2048, 256, 16, 768), 0), ((64, 2048, 256, 8, 768), 3),
-    # few experts: the rows on average decide, whatever their number
+    # few experts: the rows on average decide, and how full a round their tasks are (layer 50 -> 54 us in strips)
+    ((256, 768, 64, 8, 256), 3), ((400, 768, 64, 8, 256), DOWN), ((1792, 512, 32, 4, 256), 0),
+    ((1792, 2048, 8, 1, 256), 3),
     ((256, 512, 8, 2, 1024), 3), ((1536, 512, 8, 2, 1024), DOWN), ((975, 512, 13, 10, 384), 0),
     ((2048, 2048, 128, 8, 768), 0), ((777, 2048, 128, 8, 768), 0),
 ])
