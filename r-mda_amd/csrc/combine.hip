@@ -184,8 +184,14 @@ __device__ __forceinline__ uint4 rmda_stream_load16(const uint4 *p) {
 // output: h[r][s][c] += acc * 2 * sigmoid(inj / hc).
 //
 // What bounds it: HBM for many tokens, the chain slot -> row -> sum for few.
-// The slots and weights are scalar loads, and the streams' old values, the
-// shared row and up to KB expert rows are all in flight before the first sum.
+// The slots and weights are scalar loads, and the shared row and up to KB
+// expert rows are all in flight before the first sum.  AHEAD: so are the
+// streams' old values, for calls of few waves; with many the streams follow
+// the sum one after another, which keeps the reads and writes of a stream
+// together and 30 VGPRs free (four streams, read ahead against after: 2692
+// tokens of hidden 2048, top-2 38.7 -> 36.5 us, 1309 of hidden 1792, top-6 23.7
+// -> 23.0, 2692 of hidden 1024, top-3 23.8 -> 22.0, with the streams in the
+// Infinity Cache; 44.5 -> 43.2, 28.4 -> 26.7 and 28.8 -> 27.4 without).
 // A workgroup per token that read its slots through LDS and its rows one
 // after another took (MI355X, by events, net of the empty interval): 16
 // tokens of hidden 2560, top-10, four streams 10.7 -> 3.3 us; 128 tokens of
@@ -193,7 +199,7 @@ __device__ __forceinline__ uint4 rmda_stream_load16(const uint4 *p) {
 // (283 MB); 2048 tokens of hidden 2048 11.5 -> 11.0 us.  Single-wave workgroups
 // spread few waves over the chip, groups of four spare the dispatcher many
 // (4000 tokens of hidden 1024, top-1: 3.9 -> 3.0 us).
-template <bool HC, uint32_t KB>
+template <bool HC, uint32_t KB, bool AHEAD>
 __global__ __launch_bounds__(256) void combine16_kernel(const float *__restrict__ wt,
                                                         const uint32_t *__restrict__ slot,
                                                         const uint16_t *__restrict__ y,
@@ -217,7 +223,7 @@ __global__ __launch_bounds__(256) void combine16_kernel(const float *__restrict_
     if (wid >= waves || c >= d8) {
         return;
     }
-    constexpr uint32_t HB = 4;  // streams read ahead
+    constexpr uint32_t HB = AHEAD ? 4u : 1u;  // streams at a time
     float4 hv[HB][2];
     auto load_streams = [&](uint32_t st0) __attribute__((always_inline)) {
 #pragma unroll
@@ -229,7 +235,7 @@ __global__ __launch_bounds__(256) void combine16_kernel(const float *__restrict_
             }
         }
     };
-    if (HC) {
+    if (HC && AHEAD) {
         load_streams(0);
     }
     // the slot-scaled mode's rows stand for y * f, f a power of two: taken
@@ -278,7 +284,10 @@ __global__ __launch_bounds__(256) void combine16_kernel(const float *__restrict_
     }
     if (HC) {
         for (uint32_t st0 = 0; st0 < hcp.hc; st0 += HB) {
-            if (st0 > 0) {
+            if (!AHEAD) {
+                asm volatile("" ::: "memory");  // keeps the loads of all streams from moving up together
+            }
+            if (!AHEAD || st0 > 0) {
                 load_streams(st0);
             }
 #pragma unroll
@@ -346,14 +355,16 @@ hipError_t rmda_launch_combine16(hipStream_t s, const float *wt, const uint32_t 
         return hipSuccess;
     }
     const bool streams = hc != nullptr && hc->h != nullptr;
-    const auto kernel = streams ? (topk <= 2 ? combine16_kernel<true, 2> : combine16_kernel<true, 8>)
-                                : (topk <= 2 ? combine16_kernel<false, 2> : combine16_kernel<false, 8>);
     const uint32_t cw = (d / 8 + RMDA_WAVE - 1) / RMDA_WAVE;
     // one launch, unless its threads would not fit 32 bits
     const uint32_t most = std::max(1u, (1u << 25) / cw);
     for (uint32_t r0 = 0; r0 < rows; r0 += most) {
         const uint32_t waves = cw * std::min(most, rows - r0);
-        const uint32_t wpb = waves <= 1024 ? 1u : 4u;
+        const bool few = waves <= 1024;
+        const uint32_t wpb = few ? 1u : 4u;
+        const auto kernel = !streams ? (topk <= 2 ? combine16_kernel<false, 2, false> : combine16_kernel<false, 8, false>)
+                            : few    ? (topk <= 2 ? combine16_kernel<true, 2, true> : combine16_kernel<true, 8, true>)
+                                     : (topk <= 2 ? combine16_kernel<true, 2, false> : combine16_kernel<true, 8, false>);
         rmda_hc_t h{};
         if (streams) {
             h = *hc;
