@@ -563,6 +563,11 @@ hipError_t rmda_launch_gemm(hipStream_t s, const rmda_gemm_args_t *a);
 // 4096 row tiles; rmda_launch_gemm covers the rest.
 bool rmda_ref_mm_supported(const rmda_gemm_args_t *a);
 hipError_t rmda_launch_ref_mm(hipStream_t s, const rmda_gemm_args_t *a, uint32_t grid);
+// Whether the recording's routed GEMM of `rows` pairs takes its n192 items of up
+// to 192 rows rather than its n128 of up to 128 (ntiles column tiles, grid
+// workgroups).
+__host__ __device__ bool rmda_ref_live_tall(uint32_t n128, uint32_t n192, uint32_t ntiles, uint32_t grid,
+                                            uint32_t rows);
 #define RMDA_GEMM_BM 128u
 
 // gemm2.hip: the fused layer's grouped GEMM (SWIGLU and F16 modes) over

@@ -358,8 +358,8 @@ __global__ __launch_bounds__(768) void ref_mm_kernel(rmda_gemm_args_t g) {
 // tiles the few rows past an expert's first 128 are a task of their own (2048
 // tokens, 128 experts, top-8: half of the experts have 1 to 32 of them), so
 // every workgroup counts both kinds of items from the experts' row counts and
-// takes the height that needs less time.  Measured on MI355X: the whole
-// recording at that size 453 -> 405 us; 64 experts, 2300 tokens 388 -> 343 us;
+// takes the height that should need less time (rmda_ref_live_tall).  Measured on MI355X: the whole
+// recording at that size 453 -> 405 us; 64 experts, 2300 tokens 390 -> 355 us;
 // 16 experts top-2, 2560 x 1024, 2048 tokens 218 -> 187 us.
 //
 //   * 12 MFMA waves = 3 (M) x 4 (N) of 64 x 64 and 4 issue waves.  Up to 192
@@ -641,6 +641,28 @@ __device__ __forceinline__ void ref_live_tasks(const rmda_gemm_args_t &g, uint8_
     }
 }
 
+}  // namespace
+
+// A round costs a fixed part, its weights, and a quarter of that per 64 rows
+// of its items on average, with 12% more for a taller item's two-slot ring of
+// A.  Fitted over 171 recordings on MI355X (8 shapes of 16 to 512 experts, even
+// and skewed, rows per expert 16 to 460); summed over them this rule loses 14%
+// of one recording against always taking the better height, counting rounds
+// alone 20%.  192 rows against 128, us of the recording at 64 experts top-8,
+// 2048 x 768, gate_up and down (T: this rule takes 192): 1100 tokens T -7 and
+// T -8 of 266, 1300 T +4 and +10 of 270, 1400 T 0 and +7 of 279, 1500 T -2 and
+// T +3 of 286, 1900 T -10 and T -4 of 354, 2300 T -22 and T -10 of 404, 2700
+// +4 and T -2 of 447, 3000 +11 and T -1 of 464, 3500 +6 and T -13 of 538; equal
+// rounds up to +29 and +16 (1600).
+__host__ __device__ bool rmda_ref_live_tall(uint32_t n128, uint32_t n192, uint32_t ntiles, uint32_t grid,
+                                            uint32_t rows) {
+    const float lo = (float)((n128 * ntiles + grid - 1u) / grid) * (1.0f + (float)rows / (256.0f * (float)n128));
+    const float hi = (float)((n192 * ntiles + grid - 1u) / grid) * (1.0f + (float)rows / (256.0f * (float)n192));
+    return hi < 0.88f * lo;  // false without items
+}
+
+namespace {
+
 template <bool SWI>
 __global__ __launch_bounds__((WMW + WIW) * RMDA_WAVE) void ref_live_kernel(rmda_gemm_args_t g) {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[W_SMEM];
@@ -676,17 +698,8 @@ __global__ __launch_bounds__((WMW + WIW) * RMDA_WAVE) void ref_live_kernel(rmda_
     }
     total = __builtin_amdgcn_readfirstlane(total);
     const uint32_t ntiles = g.n_w / RN;
-    const uint32_t r_lo = ((total & 0xffffu) * ntiles + gridDim.x - 1u) / gridDim.x;
-    const uint32_t r_hi = ((total >> 16) * ntiles + gridDim.x - 1u) / gridDim.x;
-    // Rounds of either kind.  A 192-row task costs up to 1.25 (gate_up) or 1.2
-    // (down) of a 128-row one where the weights' bytes dominate, up to 1.5
-    // where the MFMAs do.  Measured on MI355X, 2048 x 768, top-8, 64 experts,
-    // 128 rows against 192: gate_up at 5 rounds against 3 (2300 tokens) -22 to
-    // -33 us of 389, 4 against 3 (1900) -11 of 352, 3 against 2 (1100) -8 of
-    // 267 and (1400) +2 of 274, 5 against 4 (3000) +14 of 464, 6 against 5
-    // (3500) +9; down at 5 against 4 (2048) -8, 6 against 4 (2600) -5, 4
-    // against 3 (1400) +8 and (1536) 0, equal rounds +5 to +7.
-    const bool tall = SWI ? 5u * r_hi < 4u * r_lo : 6u * r_hi < 5u * r_lo;
+    const bool tall = __builtin_amdgcn_readfirstlane(
+        rmda_ref_live_tall(total & 0xffffu, total >> 16, ntiles, gridDim.x, g.live_rows));
     const uint32_t sh = tall ? 16u : 0u;
     for (uint32_t c = 0; c < (ni >> sh & 0xffffu); c += 1) {
         il.e[(at >> sh & 0xffffu) + c] = (uint16_t)tid;

@@ -52,3 +52,16 @@ def strips(rows, d, experts, topk, inter, shared=0):
 ])
 def test_strip_choice(shape, want):
     assert strips(*shape) == want
+
+
+@pytest.mark.parametrize("n128,n192,ntiles,pairs,want", [
+    # 64 experts top-8, 2048 x 768 (6 gate_up tiles, 8 of down) at 1100, 1300, 1400, 1900, 2300, 2700 and 3500 tokens
+    (112, 64, 6, 8800, True), (112, 64, 8, 8800, True), (128, 65, 8, 10400, False), (128, 72, 8, 11200, False),
+    (134, 128, 6, 15200, True), (134, 128, 8, 15200, True), (191, 128, 6, 18400, True), (191, 128, 8, 18400, True),
+    (193, 129, 6, 21600, False), (193, 129, 8, 21600, True), (256, 192, 6, 28000, False), (256, 192, 8, 28000, True),
+    # equal rounds, and no items
+    (128, 107, 6, 12800, False), (128, 107, 8, 12800, False), (16, 16, 10, 1400, False), (0, 0, 8, 0, False),
+])
+def test_recording_item_height(n128, n192, ntiles, pairs, want):
+    """The measured faster height of the recording's work items, where it differs by 2 us or more."""
+    assert internal("rmda_ref_live_tall", ctypes.c_bool)(n128, n192, ntiles, 256, pairs) == want
