@@ -1763,7 +1763,7 @@ namespace {
 
 struct ShimPlan {
     size_t a16, p, idx, wt, count, off, fill, tiles, slot, xp, g, hp, hp16, ye;
-    size_t gs, hs, hs16, sh, tiles1, amax, wr, total;
+    size_t gs, hs, hs16, sh, tiles1, amax, live1, wr, total;
     uint32_t ps, rows_pad, mrows;
 };
 
@@ -1814,7 +1814,9 @@ ShimPlan plan_shim(const rmda_qwen_moe_t *q) {
         p.sh = take((size_t)p.rows_pad * d * 4);
         p.tiles1 = take((size_t)p.rows_pad / RMDA_QWEN_TILE * 4);
     }
-    p.amax = take((size_t)RMDA_QWEN_MAX_SLOTS * 4);
+    // the slots, then the shared expert's segment {offset, rows}
+    p.amax = take((size_t)(RMDA_QWEN_MAX_SLOTS + 2) * 4);
+    p.live1 = p.amax + (size_t)RMDA_QWEN_MAX_SLOTS * 4;
     // the router matrix in the packed order of the fused layer's router
     // (repacked by every recording: 2 bytes of traffic per weight byte)
     p.wr = take((size_t)d * rmda_router_cpad(p.ps) * 4);
@@ -2016,7 +2018,7 @@ int rmda_qwen_moe_rec(rmda_qwen_moe_t *q, const float *x, const float *inj, floa
     q->n_slots = 0;
     const uint32_t sx = shim_slot(q);
     uint32_t *const tiles1 = S > 0 ? scr<uint32_t>(q, p.tiles1) : nullptr;
-    uint32_t *const live1 = amax + RMDA_QWEN_MAX_SLOTS;  // {0, rows}: the words behind the slots
+    uint32_t *const live1 = scr<uint32_t>(q, p.live1);  // {0, rows}
     if (aligned(x, 16)) {
         rmda_xcast_more_t more{};
         more.zero = amax;
