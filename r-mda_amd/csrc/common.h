@@ -621,9 +621,11 @@ hipError_t rmda_launch_gemm2(hipStream_t s, const rmda_gemm_args_t *a, rmda_gemm
 // expert, 0 without one).
 // rmda_gemm_strip_items: the bound on its work items.
 // rmda_gemm_strip_waves: waves (= workgroups) of a launch.
+// rmda_gemm_strip_deep: whether they keep the deep ring.
 // rmda_gemm_strip_casts: whether down should cast the fp32 SwiGLU output
 // itself (a32).
 uint32_t rmda_gemm_strip_waves(uint32_t items, uint32_t item_rows, uint32_t n_w);
+bool rmda_gemm_strip_deep(uint32_t items, uint32_t n_w, uint32_t k);
 bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w);
 uint32_t rmda_gemm_strip_items(uint32_t npairs, uint32_t experts, uint32_t sh_rows);
 uint32_t rmda_gemm_strip_choice(uint32_t rows, uint32_t topk, uint32_t experts, uint32_t sh_rows, uint32_t inter,

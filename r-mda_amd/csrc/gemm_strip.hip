@@ -377,6 +377,12 @@ bool rmda_gemm_strip_casts(uint32_t items, uint32_t n_w) {
     return (uint64_t)items * (n_w / 32u) <= 512;
 }
 
+bool rmda_gemm_strip_deep(uint32_t items, uint32_t n_w, uint32_t k) {
+    // more waves than the chip holds at once (two per SIMD), and a K loop that
+    // fills the deep ring
+    return (uint64_t)items * (n_w / 32u) > 2048 && k >= 16 * BK;
+}
+
 hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint32_t items, uint32_t item_rows) {
     if (a->n_w % SLAB != 0 || a->k % BK != 0 || a->n_items == nullptr || a->fc.cnt != nullptr || a->ye32 != nullptr ||
         (a->a32 != nullptr && (a->mode != RMDA_GEMM_F16 || a->ye_bound == nullptr))) {
@@ -385,9 +391,7 @@ hipError_t rmda_launch_gemm_strip(hipStream_t s, const rmda_gemm_args_t *a, uint
     if (items == 0 || item_rows == 0) {
         return hipSuccess;
     }
-    // more waves than the chip holds at once (two per SIMD), and a K loop that
-    // fills the deep ring
-    const bool deep = (uint64_t)items * (a->n_w / 32u) > 2048 && a->k >= 16 * BK && a->a32 == nullptr;
+    const bool deep = a->a32 == nullptr && rmda_gemm_strip_deep(items, a->n_w, a->k);
     if (a->mode == RMDA_GEMM_SWIGLU) {
         return deep ? launch_strip<RMDA_GEMM_SWIGLU, true>(s, a, items, item_rows)
                     : launch_strip<RMDA_GEMM_SWIGLU, false>(s, a, items, item_rows);
