@@ -1233,13 +1233,18 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     float *const hp32 = x32 ? at<float>(ws, p.ye + (cast_in_down ? (size_t)p.groups_rows * d * 2 : 0)) : nullptr;
     // Streaming tile: experts averaging up to 40 rows run it with one barrier
     // per stage.  The second one keeps a fifth stage in flight, which pays
-    // while the MFMAs of a stage are long (experts of 48 rows and more) and
-    // costs more than it gives when they are short.  Layer, MI355X: 512
-    // experts top-10, hidden 2560, width 640: 10 rows 944 -> 920 us, 20 rows
-    // 1000 -> 976, 40 rows 1056 -> 1048 (from fp32 activations 1156 -> 1150),
-    // 51 rows 1237 -> 1247; hidden 2048, width 512: 20 rows 664 -> 651, 40
-    // rows 694 -> 695; 128 experts, width 768: 8 rows 213 -> 211.5, 40 rows
-    // 240 -> 241, 49 rows 247 -> 250.
+    // while the MFMAs of a stage are long and costs more than it gives when
+    // they are short.  Layer with one barrier against two (and gate_up's
+    // activation ring), MI355X, one box in turn, at 24 to 28, 31 to 36, 40, 44
+    // to 56 and 64 rows per expert:
+    //   512 experts top-10, 2560 x 640   1.00       1.00       1.00  1.00       1.03
+    //   the same from fp32 activations   0.98-0.99  0.99       0.99  0.99-1.01  1.03
+    //   512 experts top-10, 2048 x 512   1.00-1.01  1.00-1.01  1.00  1.01-1.02  1.04
+    //   128 experts top-8, 2048 x 768    1.00       1.00       1.01  1.01       1.04
+    //   256 experts top-4, 1024 x 512    0.99       0.98-0.99  0.99  0.99-1.00  1.00
+    //   64 experts top-6, 1536 x 896     0.95-0.97  0.96-0.97  1.00  0.98-1.00  1.00
+    // and with fewer rows, against two without the ring, at 10 and 20: the
+    // first shape 944 -> 920 and 1000 -> 976 us.
     rmda_gemm2_cfg_t g2 = ctx->g2;
     if (g2.spec == 6 && (uint64_t)T * K <= 40ull * E) {
         g2.spec = 4;

@@ -68,7 +68,10 @@ __global__ __launch_bounds__(256) void combine_ref_kernel(rmda_pc_moe_combine_t 
 // flight before the first sum, and y and the streams pass the caches as
 // non-temporal.  A workgroup per token that read its rows one after another
 // took (MI355X) 62 us for 2048 tokens of hidden 2048, top-8, four streams (268
-// MB), 44 us now; with the plain output 36 -> 23 us.
+// MB), 44 us now; with the plain output 36 -> 23 us.  Non-temporal pays where
+// the rows come from HBM, as they do after the GEMM that writes them (the same
+// call on three sets of buffers in turn 45 us, with ordinary accesses 55); on
+// one set, which the Infinity Cache holds, ordinary accesses take 40 us.
 template <bool HC, uint32_t KB>
 __global__ __launch_bounds__(256) void combine32_kernel(rmda_pc_moe_combine_t pc, uint32_t waves,
                                                         const float *__restrict__ wt,

@@ -1221,7 +1221,7 @@ rmda_gemm2_cfg_t rmda_gemm2_variant(int variant) {
     case 2: return {256, 32, 4, 0, 2, 0};  // the same with 4 stages
     case 3: return {256, 32, 5, 0, 0, 0};  // the same without the non-temporal weight hint
     case 4: return {256, 32, 5, 0, 2, 4};  // dedicated issue waves, one barrier per stage
-    case 5: return {256, 32, 5, 0, 2, 5};  // the default without the activation-ring switch
+    case 5: return {256, 32, 5, 0, 2, 5};  // two barriers per stage at every size, no activation ring
     case 7: return {256, 32, 5, 0, 2, 7};  // gate_up with its activation rows in a two-K-step ring
     default: return {256, 32, 5, 0, 2, 6};
     }

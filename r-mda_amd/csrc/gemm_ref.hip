@@ -359,7 +359,7 @@ __global__ __launch_bounds__(768) void ref_mm_kernel(rmda_gemm_args_t g) {
 // tokens, 128 experts, top-8: half of the experts have 1 to 32 of them), so
 // every workgroup counts both kinds of items from the experts' row counts and
 // takes the height that should need less time (rmda_ref_live_tall).  Measured on MI355X: the whole
-// recording at that size 453 -> 405 us; 64 experts, 2300 tokens 390 -> 355 us;
+// recording at that size 453 -> 405 us; 64 experts, 2300 tokens 404 -> 370 us;
 // 16 experts top-2, 2560 x 1024, 2048 tokens 218 -> 187 us.
 //
 //   * 12 MFMA waves = 3 (M) x 4 (N) of 64 x 64 and 4 issue waves.  Up to 192

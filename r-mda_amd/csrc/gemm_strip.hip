@@ -12,8 +12,8 @@
 //     contiguous KiB, so a wave loads it straight into registers, 16 bytes
 //     per lane: no LDS and no barriers.  The weights carry the non-temporal
 //     hint.
-//   * 6 to 16 K steps (by live row groups) are in flight per wave in a
-//     register ring, within 256 VGPRs so that two waves share a SIMD: 32 MB
+//   * 5 to 16 K steps (by live row groups and variant) are in flight per wave
+//     in a register ring, within 256 VGPRs so that two waves share a SIMD: 32 MB
 //     in flight over the chip against about 3 us of loaded HBM latency.  One
 //     wave per workgroup: with 4 or 8 a finished wave's registers wait for the
 //     others (one 16-token block, hidden 2048, 128 experts top-8, width 768:
@@ -360,9 +360,12 @@ uint32_t rmda_gemm_strip_choice(uint32_t rows, uint32_t topk, uint32_t experts, 
     const bool dn = strip_pays(npairs + sh_rows, groups, items, d, inter, spread);
     // One GEMM in strips keeps the other off the compute tile, which large
     // experts want: from 192 rows on average, only where the strips replace at
-    // most a quarter round of tasks (down of 13 experts of hidden 512, width
-    // 384, 176 tasks at 746 rows each: layer 60 us without, 65 with; of 8 of
-    // width 1024, 64 tasks at 384 rows: 63 and 55 us).
+    // most a quarter round of tasks.  down alone in strips, layer against the
+    // tiles by its tasks: 36 (8 experts, hidden 512, width 1024, 256 rows each)
+    // 0.78, 48 (384 rows) 0.88, 58 (512) 0.94; 76 (13 experts, 512 x 384, 384
+    // rows) 0.95, 85 (8, 1280 x 512, 224) 0.94, 94 (13, 512 rows) 1.00, 106 (20,
+    // 512 x 512, 320) 1.01, 112 (12, 1024 x 384, 256) 1.03, 120 (13, 700 rows)
+    // 1.11, 144 (12, 384 rows) 1.13.
     if (gu != dn && npairs >= 192 * experts && (uint64_t)items * ((gu ? 2 * inter : d) / SLAB) > 64) {
         return 0;
     }

@@ -6,7 +6,7 @@
 // What bounds it: HBM, every weight read and written once.  Measured on
 // MI355X, 512 experts of hidden 2560 and width 640 with a shared one, from
 // bf16 (10.1 GB moved): 2.62 -> 1.63 ms, 6.2 TB/s (a device copy reaches
-// 4.8); 12 experts of hidden 1280, width 384, also with a shared one: 43 ->
+// 5.2); 12 experts of hidden 1280, width 384, also with a shared one: 43 ->
 // 23 us.
 //   * Whole 128-byte lines on both sides: a tile's row is 256 (down: 128)
 //     columns, and 16 rows x 32 columns of a slab block are one contiguous
@@ -15,7 +15,10 @@
 //   * Small tiles in address order, loads and stores non-temporal: gate_up in
 //     tiles of 16 rows x 256 columns runs at 6.5 TB/s; 32 x 256 cost 5% more
 //     over both launches, 256 x 128 8%, 256 x 64 16%; ordinary loads 3%,
-//     ordinary stores 5%.
+//     ordinary stores 5%.  The price: the last 256 MB packed are no longer in
+//     the Infinity Cache when the first layer runs, which then takes 12 us
+//     (128 experts, 2048 x 768, 777 tokens) or 19 us (512 experts, 2048 x 512,
+//     4096 tokens) longer, once; packing these is 0.2 to 1.0 ms shorter.
 //   * The bound is summed from the tile in LDS while the next one loads, in
 //     place of a second pass over the packed down weights (0.37 ms).
 #include "common.h"
