@@ -1235,7 +1235,7 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
     // per stage.  The second one keeps a fifth stage in flight, which pays
     // while the MFMAs of a stage are long and costs more than it gives when
     // they are short.  Layer with one barrier against two (and gate_up's
-    // activation ring), MI355X, one box in turn, at 24 to 28, 31 to 36, 40, 44
+    // activation ring), MI355X, one GPU in turn, at 24 to 28, 31 to 36, 40, 44
     // to 56 and 64 rows per expert:
     //   512 experts top-10, 2560 x 640   1.00       1.00       1.00  1.00       1.03
     //   the same from fp32 activations   0.98-0.99  0.99       0.99  0.99-1.01  1.03
@@ -1320,7 +1320,7 @@ int rmda_moe_layer(rmda_moe_ctx_t *ctx, const rmda_moe_shape_t *shape, const rmd
         g.ye32 = x32 && packed == nullptr ? at<float>(ws, p.ye) : nullptr;
         g.ye_bound = x32 && packed != nullptr ? ye_bound : nullptr;
         // experts averaging 64 rows or more: either tile writes its fp16
-        // rows with non-temporal stores.  Same-box A/B: config 3 layer -1.2
+        // rows with non-temporal stores.  A/B on one GPU: config 3 layer -1.2
         // to -1.5% (down 93.6 -> 85.2 us, the combine, which then reads them
         // from HBM, 10.0 -> 12.9), config 4 (compute tile) -1.8%, config 5
         // (80 rows) -0.6 to -0.7%; at 40 rows (the teacher's shape) +0.35%

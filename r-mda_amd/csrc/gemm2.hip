@@ -50,11 +50,11 @@
 //     stage barrier instead of queueing behind MFMAs; a second barrier
 //     after the fragment reads frees a buffer before its MFMAs run, so all
 //     STAGES buffers are in flight.  Measured at config 3 against
-//     gemm2_kernel on the same boxes: gate_up 175.3 -> 172.6 us, down
+//     gemm2_kernel on the same GPUs: gate_up 175.3 -> 172.6 us, down
 //     106.1 -> 104.9 us.  The second barrier was first kept for gate_up
 //     only; with the non-temporal SwiGLU stores in place, giving it to the
 //     down GEMM as well takes the layer at config 3 from 303 to 297 us and
-//     from 289 to 286-288 us on two boxes, at config 5 from 789 to 775 and
+//     from 289 to 286-288 us on two GPUs, at config 5 from 789 to 775 and
 //     756 to 750 us, from fp32 activations at config 3 from 336 to 327-331
 //     us; configs 2 and 4 are unchanged and the teacher's shape from fp32
 //     activations 0.4% slower.  Most of the gain shows in the next call's

@@ -45,7 +45,7 @@
 //     wave computes all four of its 16-row groups: skipping the dead ones
 //     branches inside the MFMA sequence (measured on MI355X: the recording's
 //     gate_up about 7 us faster without that, 238 -> 231 and 231 -> 224 us
-//     on two boxes, its down unchanged).  At T = 2048,
+//     on two GPUs, its down unchanged).  At T = 2048,
 //     128 experts, top-8 a third of the used tiles' rows are padding.
 //   * SWI (rmda_gemm_args_t::f32_swiglu, the recording's gate_ups): the N
 //     tile is 128 gate columns j and their 128 up columns n_w/2 + j, laid out
